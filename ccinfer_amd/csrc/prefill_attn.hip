@@ -12,12 +12,12 @@
 //   1. plan kernel (one workgroup): reads query_start_loc / context_lens, emits the list of
 //      query tiles sorted longest-first (counting sort on the number of visible keys), and
 //      the list of single-token requests (decode items of a mixed batch).
-//   2. tile kernel: one workgroup (4 wavefronts) per (query tile, kv_head, head group).
-//      Each wavefront owns QW = 64 query rows of one q-head (32 for head_dim 256); the
+//   2. tile kernel: one workgroup (8 wavefronts) per (query tile, kv_head, head group).
+//      Each wavefront owns 32 query rows of one q-head (16 for head_dim 256); the
 //      workgroup covers Hq/Hkv heads that share one KV head so every K/V tile staged in LDS
 //      serves all of them. K/V tiles of 64 positions are gathered through the block table
-//      into LDS (double-buffered: the next tile's global loads are in flight while MFMAs run
-//      on the current one). Scores are formed transposed, S^T = K . Q^T, so the softmax'd
+//      into LDS (the next tiles' global loads are in flight while MFMAs run on the current
+//      one). Scores are formed transposed, S^T = K . Q^T, so the softmax'd
 //      probabilities are already in the lane layout of the P^T operand of O^T = V^T . P^T,
 //      and every O accumulator of a lane belongs to one query row (lane-local rescale).
 //      Tiles entirely above the causal diagonal are skipped; masking only runs on the
@@ -401,10 +401,13 @@ __device__ __forceinline__ bf16x8 load_vt(const __bf16* lv, int h2, int n, int l
 }
 
 // Max growth (log2 units) tolerated before the accumulators are rescaled. Probabilities
-// stay <= 2^8 and sums of them fit fp32 comfortably; acc and l always share one reference
+// stay <= 2^8 (pipelined kernel: below 2) and sums of them fit fp32 comfortably; acc and l always share one reference
 // max, so the final acc / l is exact whatever the reference.
 constexpr float kRescaleSlack = 8.0f;
 constexpr float kMaxInit = -1.0e30f;
+// Pipelined kernel: how far above a row's max the reference is set, so that probabilities
+// start at or below 2^-6 and the row may grow by 7 before one reaches 2.
+constexpr float kRefHead = 6.0f;
 
 // kPad: q / cache / output rows hold dr < D dims; the kernel runs at D with the missing dims
 // zero. kAny: any layout -- rows of any head dim dr <= D and any 2-byte alignment, cache
@@ -738,16 +741,21 @@ __global__ __launch_bounds__(kThreads) void prefill_tile_kernel(
 // MFMA: per 32-key half, S^T = K . Q^T is one 32x32 accumulator (keys x query rows) and
 // O^T += V^T . P^T runs over D/32 dim tiles x 2 key steps. Per MFMA the 32x32x16 shape
 // leaves twice the VALU issue room of the 16x16x32 one, which the softmax needs. Work
-// advances in 32-key halves through a software pipeline so that each wavefront always has
-// independent MFMA and VALU work:
-//     X_i: P_i (first key step) = exp2(S_i * scale - m)  ||  S_{i+1} = K_{i+1} . Q^T
-//     Y_i: O += V_i^T . P_i^T, with the second key step's exp beside the first PV MFMAs
-//                                                         ||  row max of S_{i+1}
-// with the instruction interleave pinned by sched_group_barrier. Masked halves seed the
-// S accumulator with 0 / -inf instead of masking the scores afterwards. K/V tiles are
-// triple-buffered in LDS: at the barrier in the middle of tile t every wavefront has
-// finished tile t-1 and tile t+1 has landed, so tile t+2 streams into the freed buffer
-// while tiles t and t+1 are read.
+// advances in 32-key halves, three stages deep, none of which waits for another of the same
+// half-step (see half_step):
+//     S(h + 2) = K . Q^T   ||   O += V(h)^T . P(h)^T   ||   P(h + 1) = exp2(S(h + 1) scale - m)
+// K and V tiles sit in rings of three in LDS, so one barrier per tile suffices and the first
+// operands of a tile's step are read before its barrier.
+//
+// What bounds it: the matrix pipe is busy 62 % of the cycles when half the CUs run (clock
+// 2.4 GHz), and the chip is power-limited (2.0-2.1 GHz) when all do. Left out one at a time in
+// copies of the kernel (1 x (12,345 cached + 1,024 new), 32q/8kv, 294 us then): LDS operand
+// reads -18 us, direct loads -20, barrier -13, row sums -14, exps -25; all but the MFMAs and
+// exps -58. Against the loop before (QK and PV in separate phases, row sums by
+// v_dot2_f32_bf16, row max in front of every exp, order left to the scheduler): that case
+// 312 -> 277 us (0.69 -> 0.78 PFLOP/s on 128 of 256 CUs), 8 x (8,192 + 1,024) 16q/8kv 548 ->
+// 518 us (1.07 -> 1.13), 8 x (512 + 1,536) 144.5 -> 141 us, head dim 64 8 x (4,096 + 1,024)
+// 350 -> 335 us, fp8 8 x (2,048 + 1,024) 195 -> 189 us.
 // ---------------------------------------------------------------------------
 template <int D>
 struct PipeShape {
@@ -793,48 +801,32 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     constexpr int kPipeRows = Sh::kRows;
     const __bf16* __restrict__ k_cache = static_cast<const __bf16*>(k_cache_v);
     const __bf16* __restrict__ v_cache = static_cast<const __bf16*>(v_cache_v);
-    // Three K/V buffers as distinct arrays (see prefill_tile_kernel: the compiler then knows
-    // the direct-to-LDS loads into one buffer never alias reads of another). fp8 uses two
-    // bf16 buffers plus two byte-staging buffers.
+    // K ring (three tiles), then V ring (three tiles). lds_dma names the same memory for the
+    // direct-to-LDS loads: taken as writes to lds_kv, each would make the compiler wait for all
+    // of them before the next read of any tile; the loop's own waits and barriers order them.
     constexpr int kTileElems = kKeysPerTile * D;
-    constexpr int kBuf2 = F8 ? 8 : kTileElems;
-    constexpr int kF8Bytes = F8 ? kTileElems : 16;
-    __shared__ __attribute__((aligned(16))) __bf16 lds_k0[kTileElems];
-    __shared__ __attribute__((aligned(16))) __bf16 lds_k1[kTileElems];
-    __shared__ __attribute__((aligned(16))) __bf16 lds_k2[kBuf2];
-    __shared__ __attribute__((aligned(16))) __bf16 lds_v0[kTileElems];
-    __shared__ __attribute__((aligned(16))) __bf16 lds_v1[kTileElems];
-    __shared__ __attribute__((aligned(16))) __bf16 lds_v2[kBuf2];
-    __shared__ __attribute__((aligned(16))) uint8_t lds_k8_0[kF8Bytes];
-    __shared__ __attribute__((aligned(16))) uint8_t lds_k8_1[kF8Bytes];
-    __shared__ __attribute__((aligned(16))) uint8_t lds_v8_0[kF8Bytes];
-    __shared__ __attribute__((aligned(16))) uint8_t lds_v8_1[kF8Bytes];
-    __shared__ uint8_t lds_valid0[kKeysPerTile];
-    __shared__ uint8_t lds_valid1[kKeysPerTile];
-    __shared__ uint8_t lds_valid2[kKeysPerTile];
+    constexpr int kTileBytes = kTileElems * 2;
+    __shared__ __attribute__((aligned(16))) __bf16 lds_kv[6 * kTileElems];
+    __shared__ __attribute__((aligned(16))) uint32_t lds_dma[4];
+    __shared__ uint8_t lds_valid[4 * kKeysPerTile];
     // The block table in LDS (fp8 staging only; the bf16 staging reads its block ids from
     // global memory into a register window).
-    __shared__ int32_t lds_bt[F8 ? kMaxTableLds : 1];
+    constexpr int kGroupMl = 2 * kPipeWaves * dcore::GroupShape<D>::kMaxG;  // decode items' (m, l)
+    __shared__ int32_t lds_bt[F8 ? kMaxTableLds : kGroupMl];
     __shared__ int s_holes[kPipeWaves];
 
     // The first dec_wgs workgroups run the batch's single-token requests instead: one per
     // (request, virtual kv head), the decode kernels' group body with prefill semantics,
-    // its partial rows in four of the bf16 K/V buffers (two wavefronts' 16 x D floats per
-    // buffer) and its (m, l) pairs in a fifth buffer.
+    // its partial rows in the K/V rings and its (m, l) pairs in the table's buffer.
     if (static_cast<int>(blockIdx.x) < dec_wgs) {
         static_assert(dcore::GroupShape<D>::kWaves == kPipeWaves &&
-                          kTileElems * 2 >= 2 * dcore::GroupShape<D>::kMaxG * D * 4 &&
-                          (F8 ? kF8Bytes : kTileElems * 2) >= 2 * kPipeWaves * 16 * 4,
-                      "the group body's partial rows fit two per K/V buffer");
+                          6 * kTileBytes >= kPipeWaves * dcore::GroupShape<D>::kMaxG * D * 4 &&
+                          kMaxTableLds >= kGroupMl,
+                      "the group body's partial rows fit the K/V rings");
         auto part = [&](int w) {
-            __bf16* b;
-            if constexpr (F8)
-                b = w < 2 ? lds_k0 : w < 4 ? lds_k1 : w < 6 ? lds_v0 : lds_v1;
-            else
-                b = w < 2 ? lds_k0 : w < 4 ? lds_k1 : w < 6 ? lds_k2 : lds_v0;
-            return reinterpret_cast<float*>(b) + (w & 1) * dcore::GroupShape<D>::kMaxG * D;
+            return reinterpret_cast<float*>(lds_kv) + w * dcore::GroupShape<D>::kMaxG * D;
         };
-        float* lm = F8 ? reinterpret_cast<float*>(lds_k8_0) : reinterpret_cast<float*>(lds_v1);
+        float* lm = reinterpret_cast<float*>(lds_bt);
         dcore::decode_group_body<D, F8, kPad, true, 0>(
             q, const_cast<void*>(k_cache_v), const_cast<void*>(v_cache_v), k_scale, v_scale,
             block_table, context_lens, out, dec_items, mbpr, hq, dec_hkv, scale_log2, dr,
@@ -933,7 +925,7 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     }
     const int64_t blk_bytes = static_cast<int64_t>(kBlock) * hkv * ds * 2;
 
-    // Per-lane LDS read offsets (elements); lane l = 32 h + c (c = l % 32, h = l / 32).
+    // Per-lane LDS read offsets (bytes); lane l = 32 h + c (c = l % 32, h = l / 32).
     // K operand of k-step kk: key row c, logical chunk 2 kk + h. Rows 16 apart share a
     // swizzle, so one offset per k-step serves both 32-key halves and every buffer.
     // V^T operand of dim tile n, k-step s: two transposing reads, of key rows
@@ -941,18 +933,18 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     // 16-lane group's 4 x 16 block, transposed so lane c receives one dim for 4 keys).
     const int c32 = lane & 31;
     const int h32 = lane >> 5;
-    int koff[S2];
+    uint32_t koff[S2];
 #pragma unroll
-    for (int kk = 0; kk < S2; ++kk) koff[kk] = lds_off<D>(c32, kk * 2 + h32);
-    int voffa[NT2], voffb[NT2];
+    for (int kk = 0; kk < S2; ++kk) koff[kk] = 2 * lds_off<D>(c32, kk * 2 + h32);
+    uint32_t voffa[NT2], voffb[NT2];
     {
         const int s16 = lane & 15;
         const int row0 = 4 * h32 + (s16 >> 2);
 #pragma unroll
         for (int n = 0; n < NT2; ++n) {
             const int dim = 32 * n + 16 * ((lane >> 4) & 1) + 4 * (s16 & 3);
-            voffa[n] = lds_off<D>(row0, dim >> 3) + (dim & 7);
-            voffb[n] = lds_off<D>(row0 + 8, dim >> 3) + (dim & 7);
+            voffa[n] = 3 * kTileBytes + 2 * (lds_off<D>(row0, dim >> 3) + (dim & 7));
+            voffb[n] = 3 * kTileBytes + 2 * (lds_off<D>(row0 + 8, dim >> 3) + (dim & 7));
         }
     }
 
@@ -966,157 +958,140 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     const __amdgpu_buffer_rsrc_t v_rsrc =
         __builtin_amdgcn_make_buffer_rsrc((void*)v_cache, 0, -1, 0x00020000);
 #endif
-    // kHoles: the table has holes in the visible range; then every tile goes through the
-    // checked path, which also records per-row validity for the mask. Otherwise only a tile
-    // that reaches past kv_end does (its rows past kv_end are zero-filled).
-    auto stage = [&](int t, __bf16* lk, __bf16* lv, uint8_t* lvalid, auto holes_tag)
-                     __attribute__((always_inline)) {
-        constexpr bool kHoles = decltype(holes_tag)::value;
-        const int key_base = t * kKeysPerTile;
-        if (t / kWin != bt_win) bt_window(t / kWin);  // wave-uniform, once per kWin tiles
-#if defined(__HIP_DEVICE_COMPILE__)
-        if (!kHoles && key_base + kKeysPerTile <= kv_end) {
-            // Buffer loads: the block's byte offset is the scalar offset, the lane's offset
-            // inside the block the vector offset (every id here fits 32 bits, see above).
-#pragma unroll
-            for (int x = 0; x < NL; ++x) {
-                const int slot0 = (x * kPipeWaves + wave) * 64;
-                const int pb = __builtin_amdgcn_readlane(btw, (t % kWin) * NL + x);
-                const int soff = pb * static_cast<int>(blk_bytes);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    k_rsrc, (__attribute__((address_space(3))) void*)(lk + slot0 * 8), 16,
-                    st_off[x], soff, 0, 0);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    v_rsrc, (__attribute__((address_space(3))) void*)(lv + slot0 * 8), 16,
-                    st_off[x], soff, 0, 0);
-            }
-            return;
+    // One matrix of one tile. A full tile (every row visible, no holes, every id within 32-bit
+    // offsets) takes buffer loads: the block's byte offset is the scalar offset, the lane's
+    // offset inside the block the vector offset. Others go through the checked path, which
+    // zero-fills rows past kv_end and in unmapped blocks (LDS holds undefined bits at
+    // workgroup start; the mask gives these rows probability 0, and 0 * V must stay finite).
+    // ids: the block ids of the tile, taken from the window when its K is staged and kept for
+    // its V, staged a step later.
+    auto tile_ids = [&](int t, int (&ids)[NL]) __attribute__((always_inline)) {
+        if (t / kWin != bt_win) {  // wave-uniform, once per kWin tiles
+            bt_window(t / kWin);
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // here, so no later use has to wait
         }
+#pragma unroll
+        for (int x = 0; x < NL; ++x) ids[x] = __builtin_amdgcn_readlane(btw, (t % kWin) * NL + x);
+    };
+    const uint32_t dma_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+        (__attribute__((address_space(3))) char*)lds_kv)) -
+        static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+            (__attribute__((address_space(3))) char*)lds_dma));
+    // LDS address for a direct load's 64 x 16 bytes: byte `off` of lds_kv, reached from lds_dma.
+    auto dma_dst = [&](int off) __attribute__((always_inline)) {
+        uint32_t o = dma_base + static_cast<uint32_t>(off);
+        asm("" : "+s"(o));
+        return (__attribute__((address_space(3))) char*)lds_dma + o;
+    };
+    auto load_full = [&](const int (&ids)[NL], bool is_k, int tile_off, int x)
+                         __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                is_k ? k_rsrc : v_rsrc,
+                (__attribute__((address_space(3))) void*)dma_dst(
+                    tile_off + (x * kPipeWaves + wave) * 64 * 16),
+                16, st_off[x], ids[x] * static_cast<int>(blk_bytes), 0, 0);
 #endif
+    };
+    auto stage_full = [&](const int (&ids)[NL], bool is_k, int tile_off)
+                          __attribute__((always_inline)) {
+#pragma unroll
+        for (int x = 0; x < NL; ++x) load_full(ids, is_k, tile_off, x);
+    };
+    auto stage_checked = [&](int t, const int (&ids)[NL], const __bf16* cache, int tile_off,
+                             uint8_t* lvalid) __attribute__((always_inline)) {
+        const int key_base = t * kKeysPerTile;
 #pragma unroll
         for (int x = 0; x < NL; ++x) {
             const int slot0 = (x * kPipeWaves + wave) * 64;
             const int row = st_row[x];
-            const int pb = __builtin_amdgcn_readlane(btw, (t % kWin) * NL + x);
-            const bool in_range = key_base + row < kv_end;
-            if (pb >= 0) {
-                const int64_t boff = static_cast<int64_t>(pb) * blk_bytes;
-                const char* kb = reinterpret_cast<const char*>(k_cache) + boff;
-                const char* vb = reinterpret_cast<const char*>(v_cache) + boff;
-                // Opaque scalar bases: keeps the address as SGPR base + 32-bit lane offset
-                // (otherwise the compiler hoists 64-bit per-lane sums out of the loop).
-                asm("" : "+s"(kb), "+s"(vb));
-                if (in_range) {
-                    __builtin_amdgcn_global_load_lds(
-                        (void*)(kb + st_off[x]),  // a char* argument makes clang drop the
-                                                  // kernel's host launch stub silently
-                        (__attribute__((address_space(3))) void*)(lk + slot0 * 8), 16, 0, 0);
-                    __builtin_amdgcn_global_load_lds(
-                        (void*)(vb + st_off[x]),
-                        (__attribute__((address_space(3))) void*)(lv + slot0 * 8), 16, 0, 0);
-                }
-            }
-            // Slots not loaded get zeros (LDS holds undefined bits at workgroup start; the
-            // mask gives these rows probability 0, and 0 * V must stay finite).
-            if (!(pb >= 0 && in_range)) {
-                *reinterpret_cast<u32x4*>(lk + (slot0 + lane) * 8) = u32x4{0, 0, 0, 0};
-                *reinterpret_cast<u32x4*>(lv + (slot0 + lane) * 8) = u32x4{0, 0, 0, 0};
-            }
-            if (kHoles && ((slot0 + lane) % CPR) == 0)
-                lvalid[row] = static_cast<uint8_t>(pb >= 0 && in_range);
+            const int pb = ids[x];
+            const bool ok = pb >= 0 && key_base + row < kv_end;
+#if defined(__HIP_DEVICE_COMPILE__)
+            // A descriptor on the block itself: 64-bit addressing, and no load of the FLAT
+            // family in the loop (those make the compiler wait for every outstanding LDS read
+            // at each use of one).
+            const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+                (void*)(reinterpret_cast<const char*>(cache) +
+                        static_cast<int64_t>(pb) * blk_bytes),
+                0, -1, 0x00020000);
+            if (ok)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    rsrc, (__attribute__((address_space(3))) void*)dma_dst(tile_off + slot0 * 16),
+                    16, st_off[x], 0, 0, 0);
+#endif
+            if (!ok)
+                *reinterpret_cast<u32x4*>(lds_kv + tile_off / 2 + (slot0 + lane) * 8) =
+                    u32x4{0, 0, 0, 0};
+            if (lvalid != nullptr && ((slot0 + lane) % CPR) == 0)
+                lvalid[row] = static_cast<uint8_t>(ok);
         }
     };
 
-    // ---- fp8 staging: tile t's bytes (16 per lane, linear in LDS) and its row scales ----
-    // Thread p (< kCh8) later converts 16-byte chunk p of the tile: row p / CPR8, dims
-    // 16 (p % CPR8) .. +16; it also fetches that row's two scales when the tile is staged.
+    // ---- fp8 staging: a tile's 16-byte chunks go through registers ----
+    // Thread p (< kCh8) owns chunk p of a tile (row p / CPR8, dims 16 (p % CPR8) .. +16): it
+    // loads the bytes and the row's scale one step ahead and converts them (byte * row scale,
+    // rounded to bf16) into the bf16 tile, in the swizzled layout the operand reads expect.
     constexpr int CPR8 = D / 16;
     constexpr int kCh8 = kKeysPerTile * CPR8;
-    constexpr int NL8 = (kCh8 + kPipeThreads - 1) / kPipeThreads;
-    const uint8_t* __restrict__ k_cache8 = static_cast<const uint8_t*>(k_cache_v);
-    const uint8_t* __restrict__ v_cache8 = static_cast<const uint8_t*>(v_cache_v);
+    static_assert(!F8 || kCh8 <= kPipeThreads, "one chunk per thread");
+    const int row8 = static_cast<int>(threadIdx.x) / CPR8;
     const int64_t blk_bytes8 = static_cast<int64_t>(kBlock) * hkv * D;
-    auto stage8 = [&](int t, uint8_t* lk8, uint8_t* lv8, uint8_t* lvalid, float& sk, float& sv)
-                      __attribute__((always_inline)) {
-        const int key_base = t * kKeysPerTile;
-#pragma unroll
-        for (int x = 0; x < NL8; ++x) {
-            const int slot0 = (x * kPipeWaves + wave) * 64;
-            if (slot0 >= kCh8) break;  // wave-uniform
-            const int p = slot0 + lane;
-            const int row = p / CPR8;
-            const int pb = __builtin_amdgcn_readfirstlane(
-                lds_bt[t * (kKeysPerTile / kBlock) + ((slot0 / CPR8) >> 4)]);
-            const bool in_range = key_base + row < kv_end;
-            if (pb >= 0 && in_range) {
-                const int64_t off = static_cast<int64_t>(pb) * blk_bytes8 +
-                                    ((row & (kBlock - 1)) * hkv + kvh) * D + (p % CPR8) * 16;
-                __builtin_amdgcn_global_load_lds(
-                    (void*)(k_cache8 + off),
-                    (__attribute__((address_space(3))) void*)(lk8 + slot0 * 16), 16, 0, 0);
-                __builtin_amdgcn_global_load_lds(
-                    (void*)(v_cache8 + off),
-                    (__attribute__((address_space(3))) void*)(lv8 + slot0 * 16), 16, 0, 0);
-            }
-            if (!(pb >= 0 && in_range)) {  // zero bytes: row scale 0 must give 0, not NaN
-                *reinterpret_cast<u32x4*>(lk8 + (slot0 + lane) * 16) = u32x4{0, 0, 0, 0};
-                *reinterpret_cast<u32x4*>(lv8 + (slot0 + lane) * 16) = u32x4{0, 0, 0, 0};
-            }
-            if ((p % CPR8) == 0) lvalid[row] = static_cast<uint8_t>(pb >= 0 && in_range);
-        }
-        sk = 0.f;
-        sv = 0.f;
-        if (static_cast<int>(threadIdx.x) < kCh8) {
-            const int row = threadIdx.x / CPR8;
-            const int pb = lds_bt[t * (kKeysPerTile / kBlock) + (row >> 4)];
-            if (pb >= 0 && key_base + row < kv_end) {
-                const int64_t si = (static_cast<int64_t>(pb) * hkv + kvh) * kBlock + (row & 15);
-                sk = k_scale[si];
-                sv = v_scale[si];
-            }
-        }
+    const uint32_t off8 = static_cast<uint32_t>(((row8 & (kBlock - 1)) * hkv + kvh) * D +
+                                                (static_cast<int>(threadIdx.x) % CPR8) * 16);
+    struct Chunk8 {
+        u32x4 w;
+        float scale;
     };
-    // Bytes of one staged tile -> bf16 tile (byte * row scale, rounded to bf16), written in
-    // the swizzled layout the operand reads expect. A row whose scale is a normal power of
-    // two (what the fp8 write stores) converts in one instruction per byte pair: the
-    // hardware's scaled conversion applies exactly the exponent of its scale operand, and
-    // byte * 2^e is exact in bf16. Any other scale takes the general path.
-    auto convert8 = [&](const uint8_t* lk8, const uint8_t* lv8, __bf16* lk, __bf16* lv,
-                        float sk, float sv) __attribute__((always_inline)) {
-        const int p = threadIdx.x;
-        if (p >= kCh8) return;
-        const int row = p / CPR8;
-        const int c = p % CPR8;
-        auto deq = [&](const uint8_t* src, __bf16* dst, float sc) __attribute__((always_inline)) {
-            const u32x4 w = *reinterpret_cast<const u32x4*>(src + p * 16);
-            u32x4 o[2];
-            const uint32_t sb = __float_as_uint(sc);
-            if ((sb & 0x007fffffu) == 0u && (sb & 0x7f800000u) != 0u) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    o[i >> 1][(i & 1) * 2] = e4m3x2_to_bf16x2<false>(w[i], sc);
-                    o[i >> 1][(i & 1) * 2 + 1] = e4m3x2_to_bf16x2<true>(w[i], sc);
-                }
-                *reinterpret_cast<u32x4*>(dst + lds_off<D>(row, 2 * c)) = o[0];
-                *reinterpret_cast<u32x4*>(dst + lds_off<D>(row, 2 * c + 1)) = o[1];
-                return;
-            }
+    auto load8 = [&](int t, const void* cache, const float* scales, uint8_t* lvalid, Chunk8& c)
+                     __attribute__((always_inline)) {
+        c.w = u32x4{0, 0, 0, 0};  // zero bytes: row scale 0 must give 0, not NaN
+        c.scale = 0.f;
+        if (kCh8 < kPipeThreads && static_cast<int>(threadIdx.x) >= kCh8) return;
+        // the chunks of a wavefront lie in one cache block
+        const int pb = __builtin_amdgcn_readfirstlane(
+            lds_bt[t * (kKeysPerTile / kBlock) + (row8 >> 4)]);
+        const bool ok = pb >= 0 && t * kKeysPerTile + row8 < kv_end;
+        if (ok) {
+            c.w = *reinterpret_cast<const u32x4*>(static_cast<const uint8_t*>(cache) +
+                                                  static_cast<int64_t>(pb) * blk_bytes8 + off8);
+            c.scale = scales[(static_cast<int64_t>(pb) * hkv + kvh) * kBlock + (row8 & 15)];
+        }
+        if (lvalid != nullptr && static_cast<int>(threadIdx.x) % CPR8 == 0)
+            lvalid[row8] = static_cast<uint8_t>(ok);
+    };
+    // A row whose scale is a normal power of two (what the fp8 write stores) converts in one
+    // instruction per byte pair: the hardware's scaled conversion applies exactly the exponent
+    // of its scale operand, and byte * 2^e is exact in bf16. Any other scale takes the general
+    // path.
+    auto convert8 = [&](const Chunk8& k, int tile_off) __attribute__((always_inline)) {
+        __bf16* dst = lds_kv + tile_off / 2;
+        if (kCh8 < kPipeThreads && static_cast<int>(threadIdx.x) >= kCh8) return;
+        const int c = static_cast<int>(threadIdx.x) % CPR8;
+        u32x4 o[2];
+        const uint32_t sb = __float_as_uint(k.scale);
+        if ((sb & 0x007fffffu) == 0u && (sb & 0x7f800000u) != 0u) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const uint32_t lo = e4m3x2_to_bf16x2<false>(w[i]);
-                const uint32_t hi = e4m3x2_to_bf16x2<true>(w[i]);
-                o[i >> 1][(i & 1) * 2] =
-                    pack_bf16x2(__uint_as_float(lo << 16) * sc, __uint_as_float(lo & 0xffff0000u) * sc);
-                o[i >> 1][(i & 1) * 2 + 1] =
-                    pack_bf16x2(__uint_as_float(hi << 16) * sc, __uint_as_float(hi & 0xffff0000u) * sc);
+                o[i >> 1][(i & 1) * 2] = e4m3x2_to_bf16x2<false>(k.w[i], k.scale);
+                o[i >> 1][(i & 1) * 2 + 1] = e4m3x2_to_bf16x2<true>(k.w[i], k.scale);
             }
-            *reinterpret_cast<u32x4*>(dst + lds_off<D>(row, 2 * c)) = o[0];
-            *reinterpret_cast<u32x4*>(dst + lds_off<D>(row, 2 * c + 1)) = o[1];
-        };
-        deq(lk8, lk, sk);
-        deq(lv8, lv, sv);
+        } else {
+            const float sc = k.scale;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t lo = e4m3x2_to_bf16x2<false>(k.w[i]);
+                const uint32_t hi = e4m3x2_to_bf16x2<true>(k.w[i]);
+                o[i >> 1][(i & 1) * 2] = pack_bf16x2(__uint_as_float(lo << 16) * sc,
+                                                     __uint_as_float(lo & 0xffff0000u) * sc);
+                o[i >> 1][(i & 1) * 2 + 1] = pack_bf16x2(__uint_as_float(hi << 16) * sc,
+                                                         __uint_as_float(hi & 0xffff0000u) * sc);
+            }
+        }
+        *reinterpret_cast<u32x4*>(dst + lds_off<D>(row8, 2 * c)) = o[0];
+        *reinterpret_cast<u32x4*>(dst + lds_off<D>(row8, 2 * c + 1)) = o[1];
     };
-    float sk8[2] = {0.f, 0.f}, sv8[2] = {0.f, 0.f};  // scales of the tiles staged in ring slot
+    [[maybe_unused]] Chunk8 k8, v8;  // the chunks in flight
 
     // Q^T operands: lane (c, h) holds dims 16 kk + 8 h .. +8 of query row tw + c.
     bf16x8 qop[S2];
@@ -1140,10 +1115,28 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     const bool holes = any_hole || nblk_vis > mbpr;
 
     // O^T: lane (c, h), element v of dim tile n holds dim 32 n + 8 (v/4) + 4 h + v%4 of
-    // query row tw + c. lsum: this lane's share of the row sum of query row tw + c (the
-    // bf16 probabilities it holds); lanes c and c + 32 together hold the whole sum.
+    // query row tw + c. lsum: the row sums of the same bf16 probabilities, on the matrix unit
+    // too: lane l holds those of query rows tw + l % 16 and + 16 in elements 0 and 1 (and
+    // again in 2 and 3).
     f32x16 acc[NT2];
-    float lsum = 0.f;
+    f32x4 lsum = {0.f, 0.f, 0.f, 0.f};
+    // Read as the B operand of the 16x16x32 MFMA, P^T operand s of the 32x32x16 one holds, in
+    // column j, the 16 keys of query row j in k-groups 0 and 2 and those of row j + 16 in
+    // groups 1 and 3. Rows of A with ones in one pair of groups sum either: one 16-cycle MFMA
+    // per 16 keys. (v_dot2_f32_bf16 runs on the matrix pipe as well: one per two 32x32x16
+    // MFMAs took that pipe from 2.0 to 1.5 PFLOP/s in a loop of both.)
+    const bf16x8 row_sel = __builtin_bit_cast(
+        bf16x8, ((lane ^ (lane >> 4)) & 1) ? u32x4{0, 0, 0, 0}
+                                           : u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
+    auto rescale = [&](float alpha) __attribute__((always_inline)) {
+        const uint32_t au = __float_as_uint(alpha);
+        // {alpha of row l % 16, alpha of row l % 16 + 16}
+        const auto pr = __builtin_amdgcn_permlane16_swap(au, au, false, false);
+        const float a0 = __uint_as_float(pr[0]), a1 = __uint_as_float(pr[1]);
+        lsum = lsum * f32x4{a0, a1, a0, a1};
+#pragma unroll
+        for (int n = 0; n < NT2; ++n) acc[n] = acc[n] * alpha;
+    };
     // A finite "no key yet" reference: exp2(s - m) needs no -inf guard, the first half with
     // a visible key always outgrows it (rescale with alpha = 0), and fully masked scores
     // (-inf) still give probability 0.
@@ -1154,27 +1147,22 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[n][v] = 0.f;
 
-    // ---- pipeline pieces (hh = 32-key half of a 64-key tile) ----
-    // S^T of one half: lane (c, h), element v holds key 8 (v/4) + 4 h + v%4 of the half.
-    // The accumulator starts at 0, or, for a masked half, at the seed mask_seed wrote
-    // (0 where visible, -inf where masked: -inf + finite products stays -inf).
-    auto qk_half = [&](const __bf16* lk, int hh, f32x16& st, auto seeded_tag)
-                       __attribute__((always_inline)) {
-        if constexpr (!decltype(seeded_tag)::value) {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) st[v] = 0.f;
-        }
-#pragma unroll
-        for (int kk = 0; kk < S2; ++kk) {
-            const bf16x8 kop = __builtin_bit_cast(
-                bf16x8, *reinterpret_cast<const u32x4*>(lk + hh * 32 * D + koff[kk]));
-            st = mfma32x32x16(kop, qop[kk], st);
-        }
-    };
+    // ---- the software pipeline over 32-key halves ----
+    // In half-step h (half h % 2 of tile h / 2) a wavefront runs, none depending on another:
+    //     S(h + 2) = K . Q^T         (S2 MFMAs, one accumulator chain)
+    //     O += V(h)^T . P(h)^T       (S2 MFMAs, NT2 chains)
+    //     P(h + 1) = exp2(S(h + 1) * scale - m), after the row max of S(h + 1)
+    // so its instruction stream alternates a QK and a PV MFMA with a quarter of the VALU
+    // work's share between each two, and every operand is read from LDS two MFMAs of its kind
+    // ahead. The order is pinned slot by slot (sched_barrier): left to the scheduler's
+    // heuristics, the same source came out as reads each waited for right before their MFMA
+    // whenever a few registers more were live. Operands read three ahead instead of two, the
+    // VALU work one slot earlier or later and the loads spread wider measured the same (+-1 %);
+    // row sums by unpacking and adding on the VALU 6 % slower.
     // Mask seed of one half (key0 = its first key): 0 for visible keys, -inf for keys past
     // the row's causal limit and, with kBits, for keys whose validity bit is clear (only
     // needed when the table has holes: otherwise every key past kv_end is past every row's
-    // limit too).
+    // limit too). S starts from the seed: -inf + finite products stays -inf.
     auto vbits_of = [&](const uint8_t* lvalid, int hh) __attribute__((always_inline)) {
         const uint64_t v = __builtin_amdgcn_ballot_w64(lvalid[lane] != 0);
         return static_cast<uint32_t>(v >> (32 * hh));
@@ -1199,285 +1187,321 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
             st[v] = ok ? 0.f : kNegInf;
         }
     };
-    // Row max of one half (scaled, log2 units); returns whether the row outgrew the slack.
-    auto max_half = [&](const f32x16& st, float& mt) __attribute__((always_inline)) {
-        float x0 = fmaxf(fmaxf(st[0], st[1]), st[2]);
-        float x1 = fmaxf(fmaxf(st[3], st[4]), st[5]);
-        float x2 = fmaxf(fmaxf(st[6], st[7]), st[8]);
-        float x3 = fmaxf(fmaxf(st[9], st[10]), st[11]);
-        float x4 = fmaxf(fmaxf(st[12], st[13]), st[14]);
-        float x = fmaxf(fmaxf(x0, x1), fmaxf(fmaxf(x2, x3), fmaxf(x4, st[15])));
-        x = wave_max_swap32(x) * scale_log2;
-        mt = x;
-        return x > m + kRescaleSlack;
+    // K operand of k-step kk of half hh (A, 32 keys x 16 dims): lane (c, h) holds key c, dims
+    // 16 kk + 8 h .. +8. S^T of a half: lane (c, h), element v holds key 8 (v/4) + 4 h + v%4.
+    // koff / voff hold the current tiles' byte addresses in lds_kv.
+    auto k_operand = [&](int hh, int kk) __attribute__((always_inline)) {
+        return __builtin_bit_cast(
+            bf16x8, *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(lds_kv) +
+                                                    hh * 32 * D * 2 + koff[kk]));
     };
-    auto rescale = [&](bool grow, const float& mt) __attribute__((always_inline)) {
-        if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-            const float m_new = fmaxf(m, mt);
-            const float alpha = __builtin_amdgcn_exp2f(m - m_new);
-            lsum = lsum * alpha;
-#pragma unroll
-            for (int n = 0; n < NT2; ++n) acc[n] = acc[n] * alpha;
-            m = m_new;
-        }
-    };
-    // P^T operands of one half: pop[s] holds elements 8 s .. 8 s + 7 (keys 16 s + 8 (e/4) +
-    // 4 h + e%4, e = 0..7), the B operand of PV k-step s. The lane's share of the row sum
-    // adds the same bf16 probabilities (v_dot2 with ones on each packed pair).
-    auto exp_part = [&](const f32x16& st, int s, bf16x8& pops) __attribute__((always_inline)) {
-        using bf16x2 = __bf16 __attribute__((ext_vector_type(2)));
-        const bf16x2 one2 = __builtin_bit_cast(bf16x2, 0x3f803f80u);
-        const float mneg = -m;
-        u32x4 pw;
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-            const float p0 =
-                __builtin_amdgcn_exp2f(__builtin_fmaf(st[8 * s + 2 * x], scale_log2, mneg));
-            const float p1 =
-                __builtin_amdgcn_exp2f(__builtin_fmaf(st[8 * s + 2 * x + 1], scale_log2, mneg));
-            const uint32_t pk = pack_bf16x2(p0, p1);
-            lsum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pk), one2, lsum,
-                                                   false);
-            pw[x] = pk;
-        }
-        pops = __builtin_bit_cast(bf16x8, pw);
-    };
-    // V^T operand (A, 32 dims x 16 keys): lane (c, h) holds dim c of the tile for keys
-    // 16 s + 4 h + r (r < 4) and 16 s + 8 + 4 h + r, matching pop[s]'s key order.
-    auto pv_part = [&](const __bf16* lv, int hh, int s, const bf16x8& pops)
-                       __attribute__((always_inline)) {
+    // V^T operand of dim tile n, k-step s (A, 32 dims x 16 keys): lane (c, h) holds dim c of
+    // the tile for keys 16 s + 4 h + r (r < 4) and 16 s + 8 + 4 h + r, matching P's key order:
+    // P^T operand s holds elements 8 s .. 8 s + 7 of S^T.
+    auto v_operand = [&](int hh, int s, int n) __attribute__((always_inline)) {
         using v4s = short __attribute__((ext_vector_type(4)));
         using v8s = short __attribute__((ext_vector_type(8)));
+        const char* base = reinterpret_cast<const char*>(lds_kv) + (hh * 32 + 16 * s) * D * 2;
+        const v4s a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) v4s*)(base + voffa[n]));
+        const v4s b = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) v4s*)(base + voffb[n]));
+        const v8s ab = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        return __builtin_bit_cast(bf16x8, ab);
+    };
+
+    // P of a half with reference m: P^T operand s holds elements 8 s .. 8 s + 7 of S^T.
+    auto exp_pair = [&](const f32x16& st, int x) __attribute__((always_inline)) {
+        return pack_bf16x2(
+            __builtin_amdgcn_exp2f(__builtin_fmaf(st[2 * x], scale_log2, -m)),
+            __builtin_amdgcn_exp2f(__builtin_fmaf(st[2 * x + 1], scale_log2, -m)));
+    };
+    // The reference a row's scores of one half ask for (log2 units).
+    auto row_ref = [&](const f32x16& st) __attribute__((always_inline)) {
+        float x = st[0];
 #pragma unroll
-        for (int n = 0; n < NT2; ++n) {
-            const __bf16* base = lv + (hh * 32 + 16 * s) * D;
-            const v4s a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) v4s*)(base + voffa[n]));
-            const v4s b = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) v4s*)(base + voffb[n]));
-            const v8s ab = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-            acc[n] = mfma32x32x16(__builtin_bit_cast(bf16x8, ab), pops, acc[n]);
+        for (int v = 1; v < 16; ++v) x = fmaxf(x, st[v]);
+        return __builtin_fmaf(wave_max_swap32(x), scale_log2, kRefHead);
+    };
+    auto exp_all = [&](const f32x16& st, bf16x8 (&p)[2]) __attribute__((always_inline)) {
+        u32x4 w[2];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) w[x >> 2][x & 3] = exp_pair(st, x);
+        p[0] = __builtin_bit_cast(bf16x8, w[0]);
+        p[1] = __builtin_bit_cast(bf16x8, w[1]);
+    };
+    bf16x8 kop[4], vop[4];  // operands read ahead (two of each kind) and the one in use
+
+    // One half-step, hh = h % 2. kQk: sq = S of half hh of the K tile (kMask: from the seed in
+    // sq); kExp: pe = P of se; always: O += V^T . pp^T over half hh of the V tile. The exps use
+    // the reference m they find, which sits kRefHead above a row's max when it is set; the check is
+    // whether any probability reached 2 (bit 14 of its bf16 form, so one OR over the packed
+    // words finds it): then m moves, and acc, the sums and P follow (acc and P always share one
+    // reference, so this is exact). The first operands are in kop / vop; those
+    // of the next half-step are read at the end (kNext), for hh = 1 from the next tiles, whose
+    // addresses turn() moves on to.
+    auto half_step = [&](auto hh_tag, f32x16& sq, f32x16& se, bf16x8 (&pe)[2],
+                         const bf16x8 (&pp)[2], auto turn, auto stage, auto qk_tag, auto exp_tag,
+                         auto mask_tag, auto next_tag) __attribute__((always_inline)) {
+        constexpr int hh = decltype(hh_tag)::value;
+        constexpr bool kNext = decltype(next_tag)::value;
+        constexpr bool kQk = decltype(qk_tag)::value;
+        constexpr bool kExp = decltype(exp_tag)::value;
+        constexpr bool kMask = decltype(mask_tag)::value;
+        constexpr int kSlots = kQk ? 2 * S2 : S2;
+        constexpr int kAhead = 2;
+        constexpr int kRing = 4;
+        static_assert(S2 % kRing == 0, "operand i of a half sits in ring position i % kRing");
+        // The last QK MFMA of the half before is two MFMAs back: its result takes about as long
+        // as two more, so the VALU work on it starts in slot kLag.
+        constexpr int kLag = kSlots >= 16 ? 3 : kSlots >= 8 ? 2 : 1;
+        constexpr int kUnits = 16;
+        float e0[8], e1[8];
+        u32x4 pw[2];
+        // VALU work in units: the exps of pair x, its packing one pair behind.
+        auto unit = [&](int j) __attribute__((always_inline)) {  // E0 E1 C0 E2 C1 ... E7 C6 C7
+            const int x = j == 0 ? 0 : j == 15 ? 7 : (j & 1) ? (j + 1) / 2 : j / 2 - 1;
+            if (j == 0 || ((j & 1) && j != 15)) {
+                e0[x] = __builtin_amdgcn_exp2f(__builtin_fmaf(se[2 * x], scale_log2, -m));
+                e1[x] = __builtin_amdgcn_exp2f(__builtin_fmaf(se[2 * x + 1], scale_log2, -m));
+            } else {
+                uint32_t pk = pack_bf16x2(e0[x], e1[x]);
+                asm volatile("" : "+v"(pk));  // stays here: not sunk past the growth branch
+                pw[x >> 2][x & 3] = pk;
+            }
+        };
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+            const int i = kQk ? s / 2 : s;
+            const bool qk = kQk && s % 2 == 0;
+            stage(s);
+            const int a = i + kAhead, an = a < S2 ? a : a - S2;
+            if (hh == 1 && a == S2) turn(qk);
+            if (a < S2 || kNext) {
+                if (qk)
+                    kop[a % kRing] = k_operand(a < S2 ? hh : 1 - hh, an);
+                else
+                    vop[a % kRing] = v_operand(a < S2 ? hh : 1 - hh, an / NT2, an % NT2);
+            }
+            if constexpr (kExp) {
+#pragma unroll
+                for (int u = 0; u < kUnits; ++u)
+                    if (kLag + u * (kSlots - kLag) / kUnits == s) unit(u);
+            }
+            if (qk) {
+                if (i == 0 && !kMask) {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) sq[v] = 0.f;
+                }
+                sq = mfma32x32x16(kop[i % kRing], qop[i], sq);
+            } else {
+                acc[i % NT2] = mfma32x32x16(vop[i % kRing], pp[i / NT2], acc[i % NT2]);
+                if (i % NT2 == 0) lsum = mfma16x16x32(row_sel, pp[i / NT2], lsum);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (kExp) {
+            pe[0] = __builtin_bit_cast(bf16x8, pw[0]);
+            pe[1] = __builtin_bit_cast(bf16x8, pw[1]);
+            const uint32_t bits = (pw[0][0] | pw[0][1] | pw[0][2]) | (pw[0][3] | pw[1][0] | pw[1][1]) |
+                                  (pw[1][2] | pw[1][3]);
+            if (__builtin_amdgcn_ballot_w64((bits & 0x40004000u) != 0) != 0) {
+                const float m_new = fmaxf(m, row_ref(se));
+                rescale(__builtin_amdgcn_exp2f(m - m_new));
+                m = m_new;
+                exp_all(se, pe);
+            }
         }
     };
 
-    // Interleave patterns for the two pipeline phases (igrouplp masks: 0x8 MFMA, 0x100 DS
-    // read, 0x402 VALU incl. transcendental). X: one QK MFMA per K read, with the exp work
-    // of the current half spread between them. Y: one PV MFMA per V^T operand (two
-    // transposing reads), with the next half's mask / max work in between.
-    constexpr int kXGroups = S2;
-    constexpr int kXValu = 3;
-    constexpr int kYValuA = 6;  // exp of the second P operand beside PV k-step 0
-    constexpr int kYValuB = 3;  // next half's row max beside PV k-step 1
-    constexpr int kXPre = 2;  // K operand reads issued ahead of the MFMAs using them
-    constexpr int kYPre = 2;  // V^T operands read ahead
-    auto interleave_x = [&]() __attribute__((always_inline)) {
-        __builtin_amdgcn_sched_group_barrier(0x100, kXPre, 0);
-#pragma unroll
-        for (int i = 0; i < kXGroups; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x402, kXValu, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (i + kXPre < kXGroups) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-    };
-    auto interleave_y = [&]() __attribute__((always_inline)) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 2 * kYPre, 0);
-#pragma unroll
-        for (int i = 0; i < 2 * NT2; ++i) {
-            if (i < NT2)
-                __builtin_amdgcn_sched_group_barrier(0x402, kYValuA, 0);
-            else
-                __builtin_amdgcn_sched_group_barrier(0x402, kYValuB, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (i + kYPre < 2 * NT2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        }
-    };
-
-    f32x16 sc;  // S of the half being exponentiated
-    f32x16 sn;  // S of the next half
-    bf16x8 pop[2];
-    float mt;
+    f32x16 s_even, s_odd;        // S of a tile's half 0 / half 1
+    bf16x8 p_even[2], p_odd[2];  // P of a tile's half 0 / half 1
+    using H0 = std::integral_constant<int, 0>;
+    using H1 = std::integral_constant<int, 1>;
+    using F = std::false_type;
+    using T = std::true_type;
+    // validity flags of a tile's rows (tables with holes): four slots, as fp8 loads run four
+    // tiles ahead of the one whose flags are read
+    auto valid_buf = [&](int t) __attribute__((always_inline)) { return lds_valid + t % 4 * kKeysPerTile; };
     // The tile loop, compiled twice: with the per-key validity bits (tables with holes) and
-    // without; each workgroup runs one of them.
-    // Whether stage(t) issues exactly 2 NL loads per wavefront (the unchecked path), so a
-    // vmcnt bound can wait for older tiles only.
-    auto full_stage = [&](int t) __attribute__((always_inline)) {
-        return !holes && t < ntiles && (t + 1) * kKeysPerTile <= kv_end;
-    };
+    // without; each workgroup runs one of them. Step t reads K of tile t + 1 and V of tile t;
+    // tile x sits in slot x % 3 of its ring. The step's barrier frees K of tile t and V of tile
+    // t - 1, whose slots take K of tile t + 3 and V of tile t + 2 (fp8: converted from
+    // registers, which then take the next chunks), and confirms what the step before staged:
+    // K of tile t + 2 and V of tile t + 1. So the first operands of step t + 1 can be read
+    // before its barrier, and no half-step starts by waiting for them.
     auto run = [&](auto holes_tag) __attribute__((always_inline)) {
-        // Prologue: tiles 0 and 1 in flight, S of tile 0 / half 0 formed, masked and maxed.
+        constexpr bool kHoles = decltype(holes_tag)::value;
+        int v_ids[NL];  // block ids of the tile whose V is staged next
+        [[maybe_unused]] int k_ids[NL];
+        const int full_tiles = kHoles ? 0 : min(ntiles, kv_end / kKeysPerTile);
+        auto stage_k = [&](int t, int off, int (&ids)[NL]) __attribute__((always_inline)) {
+            if (t >= ntiles) return;
+            tile_ids(t, ids);
+            if (t < full_tiles)
+                stage_full(ids, true, off);
+            else
+                stage_checked(t, ids, k_cache, off, kHoles ? valid_buf(t) : nullptr);
+        };
+        auto stage_v = [&](int t, int off, const int (&ids)[NL]) __attribute__((always_inline)) {
+            if (t >= ntiles) return;
+            if (t < full_tiles)
+                stage_full(ids, false, off);
+            else
+                stage_checked(t, ids, v_cache, off, nullptr);
+        };
+        auto fetch8_k = [&](int t) __attribute__((always_inline)) {
+            if (t < ntiles) load8(t, k_cache_v, k_scale, kHoles ? valid_buf(t) : nullptr, k8);
+        };
+        auto fetch8_v = [&](int t) __attribute__((always_inline)) {
+            if (t < ntiles) load8(t, v_cache_v, v_scale, nullptr, v8);
+        };
+        // S of both halves of the first tile, P of its half 0.
         if constexpr (F8) {
-            stage8(0, lds_k8_0, lds_v8_0, lds_valid0, sk8[0], sv8[0]);
-            if (ntiles > 1) stage8(1, lds_k8_1, lds_v8_1, lds_valid1, sk8[1], sv8[1]);
-            __builtin_amdgcn_s_waitcnt(0x0F70);
-            __syncthreads();
-            convert8(lds_k8_0, lds_v8_0, lds_k0, lds_v0, sk8[0], sv8[0]);
+            Chunk8 k8b;
+            fetch8_k(0);
+            fetch8_v(0);
+            k8b = k8;
+            fetch8_k(1);
+            convert8(k8b, 0);
+            convert8(v8, 3 * kTileBytes);
+            k8b = k8;
+            fetch8_k(2);
+            fetch8_v(1);
+            if (ntiles > 1) convert8(k8b, kTileBytes);
+            if (ntiles > 1) convert8(v8, 4 * kTileBytes);
+            if (ntiles > 2) convert8(k8, 2 * kTileBytes);
+            fetch8_k(3);
+            fetch8_v(2);
         } else {
-            stage(0, lds_k0, lds_v0, lds_valid0, holes_tag);
-            if (ntiles > 1) stage(1, lds_k1, lds_v1, lds_valid1, holes_tag);
-            // Tile 0 landed: vmcnt bounded by tile 1's loads when their count is exact (the
-            // checked path may issue fewer), else everything.
-            if (full_stage(1))
+            int ids0[NL], ids1[NL];
+            stage_k(0, 0, ids0);
+            stage_k(1, kTileBytes, ids1);
+            stage_v(0, 3 * kTileBytes, ids0);
+            stage_k(2, 2 * kTileBytes, v_ids);
+            stage_v(1, 4 * kTileBytes, ids1);
+            // K of tiles 0 and 1 and V of tile 0 landed: vmcnt bounded by the later loads when
+            // their count is exact, else everything.
+            if (full_tiles > 2)
                 __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * NL));
             else
                 __builtin_amdgcn_s_waitcnt(0x0F70);
         }
         __syncthreads();
-        mask_seed(sc, 0, lds_valid0, 0, holes_tag);
-        qk_half(lds_k0, 0, sc, std::true_type{});
-        const bool grow_first = max_half(sc, mt);
-        rescale(grow_first, mt);
-
-        // One tile step. Entering: sc = S of (tile t, half 0), already masked and rescaled for.
-        // kLast: tile t is the last one (no next tile to start).
-        auto step = [&](int t, auto cur, auto nxt, auto ld, auto mask_tag, auto last_tag)
-                        __attribute__((always_inline)) {
-            constexpr int BC = decltype(cur)::value;
-            constexpr int BN = decltype(nxt)::value;
-            constexpr int BL = decltype(ld)::value;
-            constexpr bool kMask = decltype(mask_tag)::value;
-            constexpr bool kLast = decltype(last_tag)::value;
-            static_assert(!F8 || (BC < 2 && BN < 2 && BL < 2), "fp8 runs a two-tile ring");
-            const __bf16* kc = BC == 0 ? lds_k0 : (BC == 1 ? lds_k1 : lds_k2);
-            const __bf16* vc = BC == 0 ? lds_v0 : (BC == 1 ? lds_v1 : lds_v2);
-            const uint8_t* valc = BC == 0 ? lds_valid0 : (BC == 1 ? lds_valid1 : lds_valid2);
-            const __bf16* kn = BN == 0 ? lds_k0 : (BN == 1 ? lds_k1 : lds_k2);
-            const uint8_t* valn = BN == 0 ? lds_valid0 : (BN == 1 ? lds_valid1 : lds_valid2);
-            __bf16* kl = BL == 0 ? lds_k0 : (BL == 1 ? lds_k1 : lds_k2);
-            __bf16* vl = BL == 0 ? lds_v0 : (BL == 1 ? lds_v1 : lds_v2);
-            uint8_t* vall = BL == 0 ? lds_valid0 : (BL == 1 ? lds_valid1 : lds_valid2);
-            const int key0 = t * kKeysPerTile;
-
-            // Halves wholly above this wavefront's last row contribute nothing: in masked
-            // steps their MFMAs and exps are skipped (wave-uniform; skip0 -> skip1 -> skipn0).
-            const int wave_lim = prefix + tw + kPipeRows - 1;
-            const bool skip0 = kMask && key0 > wave_lim;
-            const bool skip1 = kMask && key0 + 32 > wave_lim;
-            const bool skipn0 = kMask && key0 + kKeysPerTile > wave_lim;
-            auto fill_neg_inf = [](f32x16& st) __attribute__((always_inline)) {
+        {
+            mask_seed(s_even, 0, valid_buf(0), 0, holes_tag);
+            mask_seed(s_odd, 32, valid_buf(0), 1, holes_tag);
 #pragma unroll
-                for (int v = 0; v < 16; ++v) st[v] = kNegInf;
-            };
-            // X: exp of (t, 0) || QK of (t, 1)
-            __builtin_amdgcn_sched_barrier(0);
-            if (!skip1) {
-                exp_part(sc, 0, pop[0]);
-                if constexpr (kMask) mask_seed(sn, key0 + 32, valc, 1, holes_tag);
-                qk_half(kc, 1, sn, mask_tag);
-                interleave_x();
+            for (int kk = 0; kk < S2; ++kk) {
+                s_even = mfma32x32x16(k_operand(0, kk), qop[kk], s_even);
+                s_odd = mfma32x32x16(k_operand(1, kk), qop[kk], s_odd);
+            }
+            m = fmaxf(m, row_ref(s_even));
+            exp_all(s_even, p_even);
+        }
+        // Byte offsets of the ring slots, by t % 3: step t reads K of tile t + 1 and V of tile t.
+        int slot = 0;  // kTileBytes * (t % 3)
+        auto next_slot = [&](int x) __attribute__((always_inline)) {
+            return x == 2 * kTileBytes ? 0 : x + kTileBytes;
+        };
+        // The operand addresses move on one slot (K: turn(true), V: turn(false)).
+        auto turn = [&](bool is_k) __attribute__((always_inline)) {
+            const int here = is_k ? next_slot(slot) : slot;
+            const int delta = next_slot(here) - here;
+            if (is_k) {
+#pragma unroll
+                for (int kk = 0; kk < S2; ++kk) koff[kk] += delta;
             } else {
-                if (!skip0) exp_part(sc, 0, pop[0]);
-                fill_neg_inf(sn);
-            }
-            // Y: PV of (t, 0), exp of its second P operand || max of (t, 1)
-            __builtin_amdgcn_sched_barrier(0);
-            bool grow1 = false;  // skip0: S of (t, 1) is -inf, its max cannot grow
-            if (!skip0) {
-                pv_part(vc, 0, 0, pop[0]);
-                exp_part(sc, 1, pop[1]);
-                pv_part(vc, 0, 1, pop[1]);
-                grow1 = max_half(sn, mt);
-                interleave_y();
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            rescale(grow1, mt);
-            if constexpr (!kLast) {
-                __builtin_amdgcn_s_waitcnt(0x0F70);  // this wavefront's loads of tile t+1 landed
-                __syncthreads();                     // ... and everyone's; tile t-1 is free
-                if constexpr (F8) {
-                    // tile t+1: bytes (ring slot BN) -> bf16 (slot BN, which held tile t-1);
-                    // then tile t+2's bytes go to slot BL (= BC, converted one step ago)
-                    convert8(BN == 0 ? lds_k8_0 : lds_k8_1, BN == 0 ? lds_v8_0 : lds_v8_1,
-                             BN == 0 ? lds_k0 : lds_k1, BN == 0 ? lds_v0 : lds_v1, sk8[BN], sv8[BN]);
-                    __syncthreads();
-                    if (t + 2 < ntiles)
-                        stage8(t + 2, BL == 0 ? lds_k8_0 : lds_k8_1, BL == 0 ? lds_v8_0 : lds_v8_1,
-                               vall, sk8[BL], sv8[BL]);
-                } else {
-                    if (t + 2 < ntiles) stage(t + 2, kl, vl, vall, holes_tag);
+#pragma unroll
+                for (int n = 0; n < NT2; ++n) {
+                    voffa[n] += delta;
+                    voffb[n] += delta;
                 }
-            }
-            // X: exp of (t, 1) || QK of (t+1, 0)
-            __builtin_amdgcn_sched_barrier(0);
-            if (!skipn0) {
-                exp_part(sn, 0, pop[0]);
-                if constexpr (!kLast) {
-                    if constexpr (kMask)
-                        mask_seed(sc, key0 + kKeysPerTile, valn, 0, holes_tag);
-                    qk_half(kn, 0, sc, mask_tag);
-                }
-                if constexpr (!kLast) interleave_x();
-            } else {
-                if (!skip1) exp_part(sn, 0, pop[0]);
-                if constexpr (!kLast) fill_neg_inf(sc);
-            }
-            // Y: PV of (t, 1), exp of its second P operand || max of (t+1, 0)
-            __builtin_amdgcn_sched_barrier(0);
-            bool grow0 = false;  // skip1 -> skipn0: S of (t+1, 0) is -inf
-            if (!skip1) {
-                pv_part(vc, 1, 0, pop[0]);
-                exp_part(sn, 1, pop[1]);
-                pv_part(vc, 1, 1, pop[1]);
-                if constexpr (!kLast) {
-                    grow0 = max_half(sc, mt);
-                    interleave_y();
-                }
-            }
-            if constexpr (!kLast) {
-                __builtin_amdgcn_sched_barrier(0);
-                rescale(grow0, mt);
             }
         };
-        using B0 = std::integral_constant<int, 0>;
-        using B1 = std::integral_constant<int, 1>;
-        using B2 = std::integral_constant<int, 2>;
-        using F = std::false_type;
-        using T = std::true_type;
+#pragma unroll
+        for (int kk = 0; kk < S2; ++kk) koff[kk] += kTileBytes;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {  // the first operands of step 0
+            kop[i] = k_operand(0, i);
+            vop[i] = v_operand(0, i / NT2, i % NT2);
+        }
 
-        // Steps whose tiles t and t+1 lie wholly below the workgroup's first query row need no
-        // mask (unless the table has holes); they run in triples so buffer roles stay static.
-        const int mask_free_tiles = holes ? 0 : (prefix + t0 + 1) / kKeysPerTile;
-        const int mf_steps = max(0, min(ntiles - 1, mask_free_tiles - 1));
+        // The start of step t. fast: the tiles to stage are full ones.
+        auto advance = [&](int t, auto fast_tag) __attribute__((always_inline)) {
+            const int prev = next_slot(next_slot(slot));
+            if constexpr (F8) {
+                __syncthreads();
+            } else {
+                // fast: half-step 0 issues the loads, between its MFMAs
+                if constexpr (decltype(fast_tag)::value) tile_ids(t + 3, k_ids);
+                __builtin_amdgcn_s_waitcnt(0x0F70);  // this wavefront's loads have landed
+                __syncthreads();                     // ... and everyone's
+                if constexpr (!decltype(fast_tag)::value) {
+                    stage_v(t + 2, 3 * kTileBytes + prev, v_ids);
+                    stage_k(t + 3, slot, v_ids);
+                }
+            }
+        };
+        // Step t; its half-steps read ahead the first operands of the next one. kLast: no tile
+        // after t counts for this wavefront.
+        auto step = [&](int t, auto mask_tag, auto last_tag) __attribute__((always_inline)) {
+            constexpr bool kMask = decltype(mask_tag)::value;
+            constexpr bool kLast = decltype(last_tag)::value;
+            using Qk = std::integral_constant<bool, !kLast>;
+            using Seed = std::integral_constant<bool, kMask && !kLast>;
+            advance(t, std::integral_constant<bool, !kMask>{});
+            const int key1 = (t + 1) * kKeysPerTile;
+            if constexpr (Seed::value) mask_seed(s_even, key1, valid_buf(t + 1), 0, holes_tag);
+            // Staging from between the MFMAs: half-step 0 (fp8: K in half-step 0, V in 1).
+            auto stage = [&](int s) __attribute__((always_inline)) {
+                if constexpr (F8) {
+                    if (s == 1 && t + 3 < ntiles) convert8(k8, slot);
+                    if (s == 3) fetch8_k(t + 4);
+                } else if constexpr (!kMask) {
+                    if (s % 2 == 1 && s / 2 < NL)
+                        load_full(v_ids, false, 3 * kTileBytes + next_slot(next_slot(slot)), s / 2);
+                    else if (s % 2 == 1 && s / 2 < 2 * NL)
+                        load_full(k_ids, true, slot, s / 2 - NL);
+                }
+            };
+            auto stage1 = [&](int s) __attribute__((always_inline)) {
+                if constexpr (F8) {
+                    if (s == 1 && t + 2 < ntiles)
+                        convert8(v8, 3 * kTileBytes + next_slot(next_slot(slot)));
+                    if (s == 3) fetch8_v(t + 3);
+                }
+            };
+            half_step(H0{}, s_even, s_odd, p_odd, p_even, turn, stage, Qk{}, T{}, Seed{}, T{});
+            if constexpr (!F8 && !kMask) {
+#pragma unroll
+                for (int x = 0; x < NL; ++x) v_ids[x] = k_ids[x];
+            }
+            if constexpr (Seed::value) mask_seed(s_odd, key1 + 32, valid_buf(t + 1), 1, holes_tag);
+            half_step(H1{}, s_odd, s_even, p_even, p_odd, turn, stage1, Qk{}, Qk{}, Seed{}, Qk{});
+            slot = next_slot(slot);
+        };
+        // This wavefront's last tile: the ones after it lie wholly above its last row, and it
+        // only stages them.
+        const int wave_last = min(ntiles - 1, (prefix + tw + kPipeRows - 1) / kKeysPerTile);
         int t = 0;
-        if constexpr (F8) {
-            // two-tile ring: tile t in slot t % 2; the stage target of step t is slot t % 2 too
-            for (; t + 2 <= mf_steps; t += 2) {
-                step(t, B0{}, B1{}, B0{}, F{}, F{});
-                step(t + 1, B1{}, B0{}, B1{}, F{}, F{});
+        // Steps whose QK tile lies wholly below the workgroup's first query row need no mask.
+        const int mask_free_tiles = (prefix + t0 + 1) / kKeysPerTile;
+        const int fast_steps = kHoles ? 0 : min(mask_free_tiles - 1, full_tiles - 3);
+        if constexpr (!kHoles)
+            for (; t < fast_steps; ++t) step(t, F{}, F{});
+        for (; t < wave_last; ++t) step(t, T{}, F{});
+        step(t, T{}, T{});
+        for (++t; t < ntiles; ++t) {
+            advance(t, F{});
+            if constexpr (F8) {
+                if (t + 3 < ntiles) convert8(k8, slot);
+                if (t + 2 < ntiles) convert8(v8, 3 * kTileBytes + next_slot(next_slot(slot)));
+                fetch8_v(t + 3);
+                fetch8_k(t + 4);
             }
-            for (;;) {
-                if (t >= ntiles - 1) break;
-                step(t, B0{}, B1{}, B0{}, T{}, F{});
-                ++t;
-                if (t >= ntiles - 1) break;
-                step(t, B1{}, B0{}, B1{}, T{}, F{});
-                ++t;
-            }
-            if (t % 2 == 0)
-                step(t, B0{}, B1{}, B0{}, T{}, T{});
-            else
-                step(t, B1{}, B0{}, B1{}, T{}, T{});
-        } else {
-        for (; t + 3 <= mf_steps; t += 3) {
-            step(t, B0{}, B1{}, B2{}, F{}, F{});
-            step(t + 1, B1{}, B2{}, B0{}, F{}, F{});
-            step(t + 2, B2{}, B0{}, B1{}, F{}, F{});
-        }
-        for (;;) {
-            if (t >= ntiles - 1) break;
-            step(t, B0{}, B1{}, B2{}, T{}, F{});
-            ++t;
-            if (t >= ntiles - 1) break;
-            step(t, B1{}, B2{}, B0{}, T{}, F{});
-            ++t;
-            if (t >= ntiles - 1) break;
-            step(t, B2{}, B0{}, B1{}, T{}, F{});
-            ++t;
-        }
-        switch (t % 3) {
-            case 0: step(t, B0{}, B1{}, B2{}, T{}, T{}); break;
-            case 1: step(t, B1{}, B2{}, B0{}, T{}, T{}); break;
-            default: step(t, B2{}, B0{}, B1{}, T{}, T{}); break;
-        }
+            slot = next_slot(slot);
         }
     };
     if (holes)
@@ -1487,9 +1511,7 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
 
     // Epilogue: lane (c, h) holds O[tw + c][32 n + 8 i + 4 h + r] = acc[n][4 i + r].
     {
-        const float l_tot = lsum + __uint_as_float(__builtin_amdgcn_permlane32_swap(
-                                           __float_as_uint(lsum), __float_as_uint(lsum),
-                                           false, false)[h32 ? 0 : 1]);
+        const float l_tot = (lane & 16) ? lsum[1] : lsum[0];
         const int tq = tw + c32;
         if (tq < rows) {
             const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
