@@ -208,10 +208,12 @@ int prefill_entry(const void* q, const void* k_cache, const void* v_cache,
         if (err == hipSuccess) err = gather_rows(output, out_run, elems, s);
         if (err != hipSuccess) return map_hip_error(err);
     }
+    // what the workspace holds past the call's needs may take the partials of split tiles
+    const size_t used = rt.need(staged);
     const hipError_t err = prefill_attention(
         q_run, k_cache, v_cache, table, query_start_loc, context_lens, out_run, batch_size,
-        total_query_tokens, rt.mbpr16, num_q_heads, num_kv_heads, head_dim, 16, workspace, s,
-        overlap);
+        total_query_tokens, rt.mbpr16, num_q_heads, num_kv_heads, head_dim, 16, workspace,
+        ws + used, workspace_bytes - used, s, overlap);
     if (err != hipSuccess || !staged) return map_hip_error(err);
     return map_hip_error(scatter_rows(out_run, output, elems, s));
 }
@@ -244,7 +246,8 @@ int prefill_fp8_entry(const void* q, const void* k_cache, const void* v_cache,
     return map_hip_error(prefill_attention_fp8(
         q, k_cache, v_cache, k_scale, v_scale, block_table, query_start_loc, context_lens,
         output, batch_size, total_query_tokens, max_blocks_per_req, num_q_heads, num_kv_heads,
-        head_dim, workspace, as_stream(stream), overlap));
+        head_dim, workspace, static_cast<char*>(workspace) + need, workspace_bytes - need,
+        as_stream(stream), overlap));
 }
 
 }  // namespace
@@ -546,7 +549,7 @@ size_t ccinfer_prefill_workspace_size(int batch_size, int total_query_tokens,
     // the MFMA-kernel route (it covers the fp8 entry too: 16-token blocks, aligned views)
     // and the any-layout route, which a call takes for caches that are not 16-byte aligned
     // or shapes the first does not take
-    const size_t fast = rt.fast ? rt.need(true) : 0;
+    const size_t fast = rt.fast ? rt.need(true) + prefill_split_bytes(head_dim, rt.mbpr16, 16) : 0;
     const size_t any = prefill_any_supported(num_q_heads, num_kv_heads, head_dim,
                                              max_blocks_per_req)
                            ? prefill_any_workspace_bytes(batch_size, total_query_tokens,

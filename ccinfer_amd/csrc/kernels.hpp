@@ -112,6 +112,11 @@ bool prefill_fast_supported(int num_q_heads, int num_kv_heads, int head_dim,
 // The fp8 prefill (pipelined path, head_dim 64 / 128, table row staged in LDS).
 bool prefill_fp8_supported(int head_dim, int max_blocks_per_req);
 
+// Memory in which a call may keep the partial rows of split tiles (split_ws, split_bytes; at
+// any alignment); 0 where no batch of this table row splits. A call given less runs its tiles
+// whole.
+size_t prefill_split_bytes(int head_dim, int max_blocks_per_req, int block_size);
+
 size_t prefill_workspace_bytes(int batch_size, int total_query_tokens, int max_blocks_per_req,
                                int num_q_heads, int num_kv_heads, int head_dim,
                                int block_size);
@@ -129,7 +134,8 @@ hipError_t prefill_attention(const void* q, const void* k_cache, const void* v_c
                              const int32_t* context_lens, void* output, int batch_size,
                              int total_query_tokens, int max_blocks_per_req, int num_q_heads,
                              int num_kv_heads, int head_dim, int block_size, void* workspace,
-                             hipStream_t stream, const PrefillOverlap* overlap = nullptr);
+                             void* split_ws, size_t split_bytes, hipStream_t stream,
+                             const PrefillOverlap* overlap = nullptr);
 
 // ---- fp8 (OCP E4M3) KV cache, one fp32 scale per cache row -------------------------
 // Scale of (slot, kv_head) at ((slot / kFp8Block) * Hkv + kv_head) * kFp8Block + slot % 16.
@@ -157,8 +163,8 @@ hipError_t prefill_attention_fp8(const void* q, const void* k_cache, const void*
                                  const int32_t* context_lens, void* output, int batch_size,
                                  int total_query_tokens, int max_blocks_per_req,
                                  int num_q_heads, int num_kv_heads, int head_dim,
-                                 void* workspace, hipStream_t stream,
-                                 const PrefillOverlap* overlap = nullptr);
+                                 void* workspace, void* split_ws, size_t split_bytes,
+                                 hipStream_t stream, const PrefillOverlap* overlap = nullptr);
 
 // ---- per-step batch metadata built on the device ------------------------------
 constexpr int kItemDecode = 1;  // item flag: decode item (exactly one new token)

@@ -21,7 +21,9 @@
 //      probabilities are already in the lane layout of the P^T operand of O^T = V^T . P^T,
 //      and every O accumulator of a lane belongs to one query row (lane-local rescale).
 //      Tiles entirely above the causal diagonal are skipped; masking only runs on the
-//      diagonal / ragged tiles.
+//      diagonal / ragged tiles. Launches that fill at most half the CUs split the tiles' key
+//      ranges over more workgroups, whose partial rows a merge kernel combines (see "Split
+//      tiles").
 //   3. single-token requests run with prefill semantics (no 1e-6 in the denominator, bad
 //      rows left untouched). Batches (bf16 or fp8) of at most 1024 (request, virtual kv head) groups with
 //      table rows of at most 2048 positions run them in extra workgroups at the front of the
@@ -62,9 +64,30 @@ __host__ __device__ inline int heads_per_wg(int G) {
     return (G % 4 == 0) ? 4 : ((G % 2 == 0) ? 2 : 1);
 }
 
+// One workgroup's work (times the head units): query rows from t0 of request req against its
+// whole visible range.
 struct TileEntry {
     int req;
     int t0;
+};
+
+// The same where tiles may be split (see SplitPlan): against the 64-key tiles [kt0, kt1) of the
+// range. slot < 0: all of it, written to the output; else one piece, written to partial slot
+// `slot`.
+struct SplitEntry {
+    int req;
+    int t0;
+    int kt0;
+    int kt1;
+    int slot;
+};
+
+// A query tile cut into `pieces` pieces, whose partials are in slots slot0 .. + pieces.
+struct SplitTile {
+    int req;
+    int t0;
+    int slot0;
+    int pieces;
 };
 
 // Inclusive prefix sum over the 64 lanes of a wavefront (shuffles, no LDS).
@@ -110,23 +133,69 @@ __device__ void block_inclusive_scan(int* a, int n, int* part) {
 }
 
 // ---------------------------------------------------------------------------
+// Split tiles. A tile workgroup walks its whole visible range, so a launch with fewer
+// workgroups than CUs leaves CUs idle for as long as its longest tile takes. Where the batch
+// fills at most half of them, the planner cuts the longest tile into c = 256 / workgroups
+// pieces (c workgroups for every one of that size are one round of the chip), the others into
+// pieces of at most that length P, never under kSplitMinTiles. Each piece is a workgroup of its
+// own that leaves unnormalised fp32 rows and (m, l) pairs for prefill_merge_kernel.
+// A key tile takes ~1.8 us at head dim 128 (half that at 64), while a split costs the merge
+// (5-10 us) and a prologue per piece: tiles are split where that saves at least kSplitGain of
+// them. Measured, unsplit -> split: 1 x (12,345 cached + 1,024 new) 32q/8kv 280 -> 210 us, 2 x
+// (20,000 + 16) 395 -> 66, 1 x (2,000 + 512) 16q/8kv 69 -> 46, 1 x 2,048 16q/8kv 57 -> 48, 1 x
+// (900 + 200) 37.5 -> 33, fp8 1 x (8,000 + 1,024) 252 -> 166; with 176-280 workgroups (2 x
+// (1,000 + 700), 1 x 1,536 and 1 x 2,048 at 32q/8kv) pieces of unequal rounds and the merge lost
+// 6-8 us, hence the half; at savings of 8-12 key tiles the two sides are even. An estimate of
+// each of 16 piece lengths from a histogram of the pieces, on the device, found little better
+// lengths and took 5 us itself.
+// ---------------------------------------------------------------------------
+constexpr int kSplitCus = 256;
+constexpr int kSplitMinTiles = 4;
+constexpr int kSplitGain = 14;  // key tiles at head dim 128
+
+struct SplitPlan {
+    SplitTile* split;     // the split tiles (counts[2] of them)
+    SplitEntry* entries;  // the work list, in place of TileEntry's
+    int units;         // workgroups per tile; 0: tiles are not split
+    int gain;          // key tiles a split has to save
+    int key_cap;       // positions a table row can hold
+};
+
+// The piece length P for `tiles` query tiles whose longest has `longest` key tiles (a huge one:
+// no split). The host calls it with the fewest tiles and the longest table row possible, to
+// see whether a launch may split at all. At most kSplitCus / units pieces come out: every tile
+// has at most c of them.
+__host__ __device__ inline int split_length(int tiles, int units, int longest, int gain) {
+    const int wgs = tiles * units;
+    const int c = wgs > 0 ? kSplitCus / wgs : kSplitCus;
+    if (c < 2) return 0x7fffffff;
+    int P = (longest + c - 1) / c;
+    if (P < kSplitMinTiles) P = kSplitMinTiles;
+    return longest - P >= gain ? P : 0x7fffffff;
+}
+
+// ---------------------------------------------------------------------------
 // Planner: one workgroup of 1024 threads.
-// ws layout: counts[0] = #tiles, counts[1] = #decode items; tiles[max_tiles]; dec[B].
+// ws layout: counts[0] = #tile entries, counts[1] = #decode items, counts[2] = #split tiles;
+// tiles[max_tiles] (kSplit: sp.entries instead); dec[B].
 // split_dec: single-token requests become decode items (else one-row tiles).
 // kBig: more than kMaxPlanRequests requests; the per-request arrays then live in the
 // workspace (big_ntiles / big_scan, B ints each) instead of LDS.
 // ---------------------------------------------------------------------------
-template <bool kBig>
+// kSplit: tiles may be split (never with kBig); a kernel of its own, since the planner's time
+// grows with its code (one cold workgroup: +0.7 us for the split's).
+template <bool kBig, bool kSplit>
 __global__ __launch_bounds__(1024) void prefill_plan_kernel(
     const int32_t* __restrict__ qsl, const int32_t* __restrict__ context_lens, int batch_size,
     int total_tokens, int tile_tokens, int32_t* __restrict__ counts,
     TileEntry* __restrict__ tiles, int32_t* __restrict__ dec_req, uint32_t* __restrict__ zero_row,
-    int zero_words, int* __restrict__ big_ntiles, int* __restrict__ big_scan, int split_dec) {
+    int zero_words, int* __restrict__ big_ntiles, int* __restrict__ big_scan, int split_dec,
+    SplitPlan sp) {
     __shared__ int lds_ntiles[kBig ? 1 : kMaxPlanRequests];
     __shared__ int lds_scan[kBig ? 1 : kMaxPlanRequests];
-    // Each request's query length and cached prefix, read once (the bucket pass and the
+    // Each request's query rows and cached prefix, read once (the bucket pass and the
     // scatter pass need them again).
-    __shared__ int lds_qlen[kBig ? 1 : kMaxPlanRequests];
+    __shared__ int lds_rows[kBig ? 1 : kMaxPlanRequests];
     __shared__ int lds_prefix[kBig ? 1 : kMaxPlanRequests];
     int* s_ntiles = kBig ? big_ntiles : lds_ntiles;
     int* s_scan = kBig ? big_scan : lds_scan;
@@ -135,7 +204,11 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(
     __shared__ int s_part[16];
     __shared__ int s_ndec;
     __shared__ int s_total;
+    __shared__ SplitTile s_split[kSplit ? kSplitCus / 2 : 1];  // two pieces or more each
+    __shared__ int s_cost[kSplit ? kSplitCus / 2 : 1];
+    __shared__ int s_costmax, s_entries, s_slots, s_nsplit;
     const int tid = threadIdx.x;
+    if (kSplit && tid == 0) s_costmax = s_entries = s_slots = s_nsplit = 0;
     for (int i = tid; i < zero_words; i += blockDim.x) zero_row[i] = 0u;  // staging's zero row
     for (int i = tid; i < kBuckets; i += blockDim.x) s_hist[i] = 0;
     if (tid == 0) s_ndec = 0;
@@ -155,7 +228,7 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(
         const int rows = qe - (qb > 0 ? qb : 0);
         const int prefix = context_lens[b] - qlen;
         if constexpr (!kBig) {
-            lds_qlen[b] = qlen;
+            lds_rows[b] = rows;
             lds_prefix[b] = prefix;
         }
         int n = 0;
@@ -198,18 +271,51 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(
         *b_out = lo;
         *r_out = t - (s_scan[lo] - s_ntiles[lo]);
     };
-    auto bucket_of = [&](int b, int r) {
-        const int qlen = kBig ? qsl[b + 1] - qsl[b] : lds_qlen[b];
-        const int prefix = kBig ? context_lens[b] - qlen : lds_prefix[b];
+    // 64-key tiles of query tile r of request b, as the tile kernel counts them
+    auto cost_of = [&](int b, int r) {
+        int rows, prefix;
+        if constexpr (kBig) {
+            const int qb = qsl[b], qe = qsl[b + 1];
+            rows = (qe < total_tokens ? qe : total_tokens) - qb;
+            prefix = context_lens[b] - (qe - qb);
+        } else {
+            rows = lds_rows[b];
+            prefix = lds_prefix[b];
+        }
         int last = (r + 1) * tile_tokens;
-        if (last > qlen) last = qlen;
-        const int cost = (prefix + last) >> 6;
+        if (last > rows) last = rows;
+        const int keys = min(prefix + last, sp.key_cap);
+        return (keys + kKeysPerTile - 1) / kKeysPerTile;
+    };
+    auto bucket_of = [&](int cost) {
         return kBuckets - 1 - (cost < kBuckets - 1 ? cost : kBuckets - 1);
     };
+    int P = 0x7fffffff;  // key tiles a piece may have
+    if constexpr (kSplit) {
+        int c = 0;
+        for (int t = tid; t < total; t += blockDim.x) {
+            int b, r;
+            locate(t, &b, &r);
+            c = max(c, cost_of(b, r));
+        }
+        if (c > 0) atomicMax(&s_costmax, c);
+        __syncthreads();
+        P = split_length(total, sp.units, s_costmax, sp.gain);
+    }
+    // A split tile's first cost % c pieces have cost / c + 1 key tiles, the others cost / c.
     for (int t = tid; t < total; t += blockDim.x) {
         int b, r;
         locate(t, &b, &r);
-        atomicAdd(&s_hist[bucket_of(b, r)], 1);
+        const int cost = cost_of(b, r);
+        if (!kSplit || cost <= P) {
+            atomicAdd(&s_hist[bucket_of(cost)], 1);
+        } else {
+            const int c = (cost + P - 1) / P;
+            const int len = cost / c, more = cost - len * c;
+            if (more > 0) atomicAdd(&s_hist[bucket_of(len + 1)], more);
+            atomicAdd(&s_hist[bucket_of(len)], c - more);
+            atomicAdd(&s_entries, c - 1);
+        }
     }
     __syncthreads();
     // Exclusive scan of the histogram -> first slot of each bucket.
@@ -221,12 +327,40 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(
     for (int t = tid; t < total; t += blockDim.x) {
         int b, r;
         locate(t, &b, &r);
-        const int pos = atomicAdd(&s_hist[bucket_of(b, r)], 1);
-        tiles[pos] = TileEntry{b, r * tile_tokens};
+        const int cost = cost_of(b, r);
+        if (!kSplit || cost <= P) {
+            const int pos = atomicAdd(&s_hist[bucket_of(cost)], 1);
+            if (kSplit)
+                sp.entries[pos] = SplitEntry{b, r * tile_tokens, 0, cost, -1};
+            else
+                tiles[pos] = TileEntry{b, r * tile_tokens};
+        } else {
+            const int c = (cost + P - 1) / P;
+            const int i = atomicAdd(&s_nsplit, 1);
+            const SplitTile st{b, r * tile_tokens, atomicAdd(&s_slots, c), c};
+            sp.split[i] = st;
+            s_split[i] = st;
+            s_cost[i] = cost;
+        }
+    }
+    if constexpr (kSplit) {
+        __syncthreads();
+        // one wavefront per split tile, one lane per piece
+        for (int i = tid >> 6; i < s_nsplit; i += blockDim.x >> 6) {
+            const SplitTile st = s_split[i];
+            const int len = s_cost[i] / st.pieces, more = s_cost[i] - len * st.pieces;
+            for (int k = tid & 63; k < st.pieces; k += 64) {
+                const int k0 = k * len + min(k, more);
+                const int size = len + (k < more ? 1 : 0);
+                const int pos = atomicAdd(&s_hist[bucket_of(size)], 1);
+                sp.entries[pos] = SplitEntry{st.req, st.t0, k0, k0 + size, st.slot0 + k};
+            }
+        }
     }
     if (tid == 0) {
-        counts[0] = total;
+        counts[0] = total + (kSplit ? s_entries : 0);
         counts[1] = s_ndec;
+        if (kSplit) counts[2] = s_nsplit;
     }
 }
 
@@ -788,7 +922,8 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
                          const int32_t* __restrict__ counts, const TileEntry* __restrict__ tiles,
                          int total_tokens, int mbpr, int hq, int hkv, float scale_log2,
                          int dr, dcore::ItemArgs dec_items, int dec_wgs, int dec_hkv,
-                         int dec_rep) {
+                         int dec_rep, const SplitEntry* __restrict__ entries,
+                         float* __restrict__ part_o, float* __restrict__ part_ml) {
     static_assert(!(F8 && kPad), "fp8 runs the native head dims only");
     const int ds = kPad ? dr : D;  // row stride of q / cache / output (elements)
     using Sh = PipeShape<D>;
@@ -844,7 +979,14 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     const int u = bid % U;
     const int kvh = u / (G / HPW);
     const int hg = u % (G / HPW);
-    const TileEntry te = tiles[tile_idx];
+    SplitEntry te{0, 0, 0, 0x7fffffff, -1};
+    if (entries != nullptr) {
+        te = entries[tile_idx];
+    } else {
+        const TileEntry whole = tiles[tile_idx];
+        te.req = whole.req;
+        te.t0 = whole.t0;
+    }
     const int req = te.req;
     const int t0 = te.t0;
 
@@ -858,7 +1000,9 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     const int kv_end = prefix + min(t0 + TT, rows);  // keys past it are masked for every row
     // Positions past the table row are invalid: no tile needs to reach them.
     const int kv_lim = min(kv_end, mbpr * kBlock);
-    const int ntiles = (kv_lim + kKeysPerTile - 1) / kKeysPerTile;
+    // This workgroup's key tiles [kt0, ntiles): the whole range, or one piece of it.
+    const int kt0 = te.kt0;
+    const int ntiles = min(te.kt1, (kv_lim + kKeysPerTile - 1) / kKeysPerTile);
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -884,7 +1028,7 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
         bt_win = win;
     };
     // The first window's load goes out before the table scan below, so the two overlap.
-    if constexpr (!F8) bt_window(0);
+    if constexpr (!F8) bt_window(kt0 / kWin);
 
     // Block-table slice in LDS (fp8): entries for every block the tiles touch, -1 past the
     // visible range or the table row. Holes (negative ids inside the visible range, or a
@@ -896,10 +1040,12 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
         min(static_cast<int64_t>(0x7fffffff),
             static_cast<int64_t>(0xffffffffll / (static_cast<int64_t>(kBlock) * hkv * ds * 2)) - 1));
     bool bad = false;
-    for (int lb = threadIdx.x; lb < (F8 ? ntiles * (kKeysPerTile / kBlock) : nblk);
-         lb += kPipeThreads) {
+    constexpr int kTileBlocks = kKeysPerTile / kBlock;
+    const int lb_first = kt0 * kTileBlocks;
+    for (int lb = lb_first + static_cast<int>(threadIdx.x);
+         lb < (F8 ? ntiles * kTileBlocks : min(nblk, ntiles * kTileBlocks)); lb += kPipeThreads) {
         const int pb = lb < nblk ? req_blocks[lb] : -1;
-        if constexpr (F8) lds_bt[lb] = pb;
+        if constexpr (F8) lds_bt[lb - lb_first] = pb;
         bad = bad || (lb < nblk && (pb < 0 || pb > max_fast_pb));
     }
     {
@@ -1050,7 +1196,7 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
         if (kCh8 < kPipeThreads && static_cast<int>(threadIdx.x) >= kCh8) return;
         // the chunks of a wavefront lie in one cache block
         const int pb = __builtin_amdgcn_readfirstlane(
-            lds_bt[t * (kKeysPerTile / kBlock) + (row8 >> 4)]);
+            lds_bt[(t - kt0) * kTileBlocks + (row8 >> 4)]);
         const bool ok = pb >= 0 && t * kKeysPerTile + row8 < kv_end;
         if (ok) {
             c.w = *reinterpret_cast<const u32x4*>(static_cast<const uint8_t*>(cache) +
@@ -1326,7 +1472,7 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     auto valid_buf = [&](int t) __attribute__((always_inline)) { return lds_valid + t % 4 * kKeysPerTile; };
     // The tile loop, compiled twice: with the per-key validity bits (tables with holes) and
     // without; each workgroup runs one of them. Step t reads K of tile t + 1 and V of tile t;
-    // tile x sits in slot x % 3 of its ring. The step's barrier frees K of tile t and V of tile
+    // tile x sits in slot (x - kt0) % 3 of its ring. The step's barrier frees K of tile t and V of tile
     // t - 1, whose slots take K of tile t + 3 and V of tile t + 2 (fp8: converted from
     // registers, which then take the next chunks), and confirms what the step before staged:
     // K of tile t + 2 and V of tile t + 1. So the first operands of step t + 1 can be read
@@ -1360,38 +1506,38 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
         // S of both halves of the first tile, P of its half 0.
         if constexpr (F8) {
             Chunk8 k8b;
-            fetch8_k(0);
-            fetch8_v(0);
+            fetch8_k(kt0);
+            fetch8_v(kt0);
             k8b = k8;
-            fetch8_k(1);
+            fetch8_k(kt0 + 1);
             convert8(k8b, 0);
             convert8(v8, 3 * kTileBytes);
             k8b = k8;
-            fetch8_k(2);
-            fetch8_v(1);
-            if (ntiles > 1) convert8(k8b, kTileBytes);
-            if (ntiles > 1) convert8(v8, 4 * kTileBytes);
-            if (ntiles > 2) convert8(k8, 2 * kTileBytes);
-            fetch8_k(3);
-            fetch8_v(2);
+            fetch8_k(kt0 + 2);
+            fetch8_v(kt0 + 1);
+            if (kt0 + 1 < ntiles) convert8(k8b, kTileBytes);
+            if (kt0 + 1 < ntiles) convert8(v8, 4 * kTileBytes);
+            if (kt0 + 2 < ntiles) convert8(k8, 2 * kTileBytes);
+            fetch8_k(kt0 + 3);
+            fetch8_v(kt0 + 2);
         } else {
             int ids0[NL], ids1[NL];
-            stage_k(0, 0, ids0);
-            stage_k(1, kTileBytes, ids1);
-            stage_v(0, 3 * kTileBytes, ids0);
-            stage_k(2, 2 * kTileBytes, v_ids);
-            stage_v(1, 4 * kTileBytes, ids1);
-            // K of tiles 0 and 1 and V of tile 0 landed: vmcnt bounded by the later loads when
+            stage_k(kt0, 0, ids0);
+            stage_k(kt0 + 1, kTileBytes, ids1);
+            stage_v(kt0, 3 * kTileBytes, ids0);
+            stage_k(kt0 + 2, 2 * kTileBytes, v_ids);
+            stage_v(kt0 + 1, 4 * kTileBytes, ids1);
+            // K of the first two tiles and V of the first landed: vmcnt bounded by the later loads when
             // their count is exact, else everything.
-            if (full_tiles > 2)
+            if (kt0 + 2 < full_tiles)
                 __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * NL));
             else
                 __builtin_amdgcn_s_waitcnt(0x0F70);
         }
         __syncthreads();
         {
-            mask_seed(s_even, 0, valid_buf(0), 0, holes_tag);
-            mask_seed(s_odd, 32, valid_buf(0), 1, holes_tag);
+            mask_seed(s_even, kt0 * kKeysPerTile, valid_buf(kt0), 0, holes_tag);
+            mask_seed(s_odd, kt0 * kKeysPerTile + 32, valid_buf(kt0), 1, holes_tag);
 #pragma unroll
             for (int kk = 0; kk < S2; ++kk) {
                 s_even = mfma32x32x16(k_operand(0, kk), qop[kk], s_even);
@@ -1400,8 +1546,8 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
             m = fmaxf(m, row_ref(s_even));
             exp_all(s_even, p_even);
         }
-        // Byte offsets of the ring slots, by t % 3: step t reads K of tile t + 1 and V of tile t.
-        int slot = 0;  // kTileBytes * (t % 3)
+        // Byte offsets of the ring slots: step t reads K of tile t + 1 and V of tile t.
+        int slot = 0;  // kTileBytes * ((t - kt0) % 3)
         auto next_slot = [&](int x) __attribute__((always_inline)) {
             return x == 2 * kTileBytes ? 0 : x + kTileBytes;
         };
@@ -1423,7 +1569,7 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
 #pragma unroll
         for (int kk = 0; kk < S2; ++kk) koff[kk] += kTileBytes;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {  // the first operands of step 0
+        for (int i = 0; i < 2; ++i) {  // the first operands of the first step
             kop[i] = k_operand(0, i);
             vop[i] = v_operand(0, i / NT2, i % NT2);
         }
@@ -1484,8 +1630,9 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
         };
         // This wavefront's last tile: the ones after it lie wholly above its last row, and it
         // only stages them.
-        const int wave_last = min(ntiles - 1, (prefix + tw + kPipeRows - 1) / kKeysPerTile);
-        int t = 0;
+        const int wave_last =
+            max(kt0, min(ntiles - 1, (prefix + tw + kPipeRows - 1) / kKeysPerTile));
+        int t = kt0;
         // Steps whose QK tile lies wholly below the workgroup's first query row need no mask.
         const int mask_free_tiles = (prefix + t0 + 1) / kKeysPerTile;
         const int fast_steps = kHoles ? 0 : min(mask_free_tiles - 1, full_tiles - 3);
@@ -1512,6 +1659,21 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     // Epilogue: lane (c, h) holds O[tw + c][32 n + 8 i + 4 h + r] = acc[n][4 i + r].
     {
         const float l_tot = (lane & 16) ? lsum[1] : lsum[0];
+        if (te.slot >= 0) {
+            // A piece of a split tile: the lanes' accumulators as they are, 16 bytes a lane
+            // and store (a row-major layout would scatter them), for prefill_merge_kernel.
+            const int64_t wv = (static_cast<int64_t>(te.slot) * U + u) * kPipeWaves + wave;
+            f32x4* po = reinterpret_cast<f32x4*>(part_o) + wv * (NT2 * 4 * 64) + lane;
+#pragma unroll
+            for (int n = 0; n < NT2; ++n)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    po[(n * 4 + i) * 64] = f32x4{acc[n][4 * i], acc[n][4 * i + 1],
+                                                 acc[n][4 * i + 2], acc[n][4 * i + 3]};
+            if (h32 == 0)
+                *reinterpret_cast<f32x2*>(part_ml + (wv * kPipeRows + c32) * 2) = f32x2{m, l_tot};
+            return;
+        }
         const int tq = tw + c32;
         if (tq < rows) {
             const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
@@ -1531,12 +1693,91 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     }
 }
 
+// Log-sum-exp merge of the pieces of split tiles (counts[2] of them). One wavefront per
+// (split tile, unit, wavefront of the tile kernel, 32-dim block n): it reads the partials in
+// the tile kernel's own lane layout, so every load is a whole kilobyte, and stores the rows as
+// that kernel's epilogue does.
+template <int D, bool kPad>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(
+    __bf16* __restrict__ out, const float* __restrict__ part_o,
+    const float* __restrict__ part_ml, const int32_t* __restrict__ counts,
+    const SplitTile* __restrict__ split, const int32_t* __restrict__ qsl, int total_tokens,
+    int hq, int hkv, int dr) {
+    constexpr int kPipeWaves = PipeShape<D>::kWaves;
+    constexpr int kPipeRows = PipeShape<D>::kRows;
+    constexpr int NT2 = D / 32;
+    const int ds = kPad ? dr : D;
+    const int G = hq / hkv;
+    const int HPW = heads_per_wg(G);
+    const int WPH = kPipeWaves / HPW;
+    const int U = hkv * (G / HPW);
+    const int lane = threadIdx.x & 63;
+    const int wi = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = wi % NT2;
+    const int wave = wi / NT2 % kPipeWaves;
+    const int u = wi / (NT2 * kPipeWaves) % U;
+    const int si = wi / (NT2 * kPipeWaves * U);
+    if (si >= counts[2]) return;
+    const SplitTile st = split[si];
+    const int qb = qsl[st.req];
+    const int rows = min(qsl[st.req + 1], total_tokens) - qb;
+    const int tw = st.t0 + (wave % WPH) * kPipeRows;
+    if (tw >= rows) return;
+    const int q_head = u / (G / HPW) * G + u % (G / HPW) * HPW + wave / WPH;
+    const int c32 = lane & 31;
+    const int h32 = lane >> 5;
+    const int64_t wv0 = (static_cast<int64_t>(st.slot0) * U + u) * kPipeWaves + wave;
+    const int64_t step = static_cast<int64_t>(U) * kPipeWaves;
+    float mmax = kMaxInit;
+#pragma unroll 8
+    for (int p = 0; p < st.pieces; ++p)
+        mmax = fmaxf(mmax, part_ml[((wv0 + p * step) * kPipeRows + c32) * 2]);
+    f32x4 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float l = 0.f;
+#pragma unroll 4
+    for (int p = 0; p < st.pieces; ++p) {
+        const int64_t wv = wv0 + p * step;
+        const f32x2 ml = *reinterpret_cast<const f32x2*>(part_ml + (wv * kPipeRows + c32) * 2);
+        const f32x4* po = reinterpret_cast<const f32x4*>(part_o) + wv * (NT2 * 4 * 64) +
+                          n * 4 * 64 + lane;
+        const float w = __builtin_amdgcn_exp2f(ml[0] - mmax);
+        l += ml[1] * w;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = acc[i] + po[i * 64] * w;
+    }
+    const int tq = tw + c32;
+    if (tq >= rows) return;
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    __bf16* o = out + (static_cast<int64_t>(qb + tq) * hq + q_head) * ds;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (kPad && 32 * n + 8 * i + 4 * h32 >= dr) continue;  // padded dims
+        u32x2 w;
+        w[0] = pack_bf16x2(acc[i][0] * inv, acc[i][1] * inv);
+        w[1] = pack_bf16x2(acc[i][2] * inv, acc[i][3] * inv);
+        *reinterpret_cast<u32x2*>(o + 32 * n + 8 * i + 4 * h32) = w;
+    }
+}
+
 struct PrefillLayout {
     size_t counts_off, zero_off, tiles_off, dec_off, big_off, decode_ws_off, total;
     int max_tiles;
     int tile_tokens;
+    int units;   // workgroups per query tile
+    int gain;    // key tiles a split has to save
+    bool split;  // whether the planner may split tiles (given the memory for it)
     DecodePlan plan;
 };
+
+int split_gain(int D) { return D <= 64 ? 2 * kSplitGain : kSplitGain; }
+
+// 64-key tiles a table row can hold (block counts times sizes fit an int).
+int row_key_tiles(int max_blocks_per_req, int block_size) {
+    return static_cast<int>(
+        (static_cast<int64_t>(max_blocks_per_req) * block_size + kKeysPerTile - 1) / kKeysPerTile);
+}
 
 size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
@@ -1554,11 +1795,21 @@ PrefillLayout prefill_layout(int batch_size, int total_query_tokens, int max_blo
     const int D = decode_mfma_dim(head_dim);  // the kernels' (padded) head dim
     L.tile_tokens = tile_tokens_for(D, G);
     L.max_tiles = total_query_tokens / L.tile_tokens + batch_size;
+    L.units = num_kv_heads * (G / heads_per_wg(G));
+    // Whether the planner may split tiles: the same rule for the fewest tiles these tokens can
+    // make (at least one a request: single-token requests make none, but a batch that has
+    // many of those is not short of workgroups) and a table row full of positions. A split is
+    // then possible, not certain.
+    L.gain = split_gain(D);
+    if (pipe_head_dim(D) && batch_size <= kMaxPlanRequests &&
+        split_length(std::max(batch_size, total_query_tokens / L.tile_tokens), L.units,
+                     row_key_tiles(max_blocks_per_req, block_size), L.gain) < 0x7fffffff)
+        L.split = true;
     L.plan = plan_decode_items(batch_size, num_q_heads, num_kv_heads, head_dim,
                                max_blocks_per_req * block_size, fp8);
     size_t off = 0;
     L.counts_off = off;
-    off = align256(off + 2 * sizeof(int32_t));
+    off = align256(off + 3 * sizeof(int32_t));
     L.zero_off = off;  // one all-zero K/V row (D bf16), rewritten by the planner
     off = align256(off + static_cast<size_t>(D) * 2);
     L.tiles_off = off;
@@ -1574,6 +1825,14 @@ PrefillLayout prefill_layout(int batch_size, int total_query_tokens, int max_blo
     return L;
 }
 
+// The memory of split tiles: their list, the work list (a batch that may split has at most
+// kSplitCus / 2 requests and as many whole tiles of its tokens, and kSplitCus pieces), then
+// the partial rows and (m, l) pairs of at most kSplitCus workgroups.
+constexpr size_t kSplitListBytes =
+    (kSplitCus / 2 * sizeof(SplitTile) + 2 * kSplitCus * sizeof(SplitEntry) + 255) & ~size_t{255};
+constexpr size_t kSplitRows =
+    static_cast<size_t>(kSplitCus) * PipeShape<64>::kWaves * PipeShape<64>::kRows;
+
 // dr: the head dim of q / cache / output rows (dr == D unless kPad).
 template <int D, bool F8, bool kPad>
 hipError_t launch_tiles(const void* q, const void* k_cache, const void* v_cache,
@@ -1582,7 +1841,8 @@ hipError_t launch_tiles(const void* q, const void* k_cache, const void* v_cache,
                         const int32_t* context_lens, void* output, int total_query_tokens,
                         int mbpr, int hq, int hkv, int block_size, const int32_t* counts,
                         const TileEntry* tiles, const void* zero_row, int max_tiles,
-                        hipStream_t stream, int dr, int batch_size, bool fused_dec) {
+                        hipStream_t stream, int dr, int batch_size, bool fused_dec,
+                        const SplitPlan& sp, float* part_o, float* part_ml) {
     const int G = hq / hkv;
     const int U = hkv * (G / heads_per_wg(G));
     const float scale_log2 = kLog2e / sqrtf(static_cast<float>(dr));
@@ -1599,13 +1859,23 @@ hipError_t launch_tiles(const void* q, const void* k_cache, const void* v_cache,
             it.singles_total = total_query_tokens;
             dec_wgs = batch_size * hkv * rep;
         }
-        const int64_t grid = static_cast<int64_t>(max_tiles) * U + dec_wgs;
+        const int max_entries = max_tiles + (sp.units > 0 ? kSplitCus / sp.units : 0);
+        const int64_t grid = static_cast<int64_t>(max_entries) * U + dec_wgs;
         prefill_pipe_kernel<D, F8, kPad>
             <<<static_cast<unsigned>(grid), PipeShape<D>::kThreads, 0, stream>>>(
             static_cast<const __bf16*>(q), k_cache, v_cache, k_scale, v_scale, block_table, qsl,
             context_lens,
             static_cast<__bf16*>(output), counts, tiles, total_query_tokens, mbpr, hq, hkv,
-            scale_log2, dr, it, dec_wgs, hkv * rep, rep);
+            scale_log2, dr, it, dec_wgs, hkv * rep, rep,
+            sp.units > 0 ? sp.entries : nullptr, part_o, part_ml);
+        const hipError_t err = hipGetLastError();
+        if (err != hipSuccess || sp.units == 0) return err;
+        // four wavefronts a workgroup; a tile has 8 D / 32 U of them (a multiple of four)
+        const int64_t mwgs = static_cast<int64_t>(std::min(max_tiles, kSplitCus / 2 / U)) * U *
+                             (PipeShape<D>::kWaves * (D / 32) / 4);
+        prefill_merge_kernel<D, kPad><<<static_cast<unsigned>(mwgs), 256, 0, stream>>>(
+            static_cast<__bf16*>(output), part_o, part_ml, counts, sp.split, qsl,
+            total_query_tokens, hq, hkv, dr);
         return hipGetLastError();
     } else if constexpr (F8) {
         return hipErrorInvalidValue;  // fp8 has the pipelined path only
@@ -1635,6 +1905,14 @@ bool prefill_fast_supported(int num_q_heads, int num_kv_heads, int head_dim,
 
 bool prefill_fp8_supported(int head_dim, int max_blocks_per_req) {
     return pipe_head_dim(head_dim) && max_blocks_per_req <= kMaxTableLds;
+}
+
+size_t prefill_split_bytes(int head_dim, int max_blocks_per_req, int block_size) {
+    const int D = decode_mfma_dim(head_dim);
+    if (!pipe_head_dim(D) ||
+        row_key_tiles(max_blocks_per_req, block_size) < kSplitMinTiles + split_gain(D))
+        return 0;
+    return 256 + kSplitListBytes + kSplitRows * (D + 2) * sizeof(float);
 }
 
 size_t prefill_workspace_bytes(int batch_size, int total_query_tokens, int max_blocks_per_req,
@@ -1683,8 +1961,8 @@ hipError_t prefill_impl(const void* q, const void* k_cache, const void* v_cache,
                         const int32_t* query_start_loc, const int32_t* context_lens,
                         void* output, int batch_size, int total_query_tokens,
                         int max_blocks_per_req, int num_q_heads, int num_kv_heads, int head_dim,
-                        int block_size, void* workspace, hipStream_t stream,
-                        const PrefillOverlap* overlap) {
+                        int block_size, void* workspace, void* split_ws, size_t split_bytes,
+                        hipStream_t stream, const PrefillOverlap* overlap) {
     const PrefillLayout L = prefill_layout(batch_size, total_query_tokens, max_blocks_per_req,
                                            num_q_heads, num_kv_heads, head_dim, block_size, F8);
     char* ws = static_cast<char*>(workspace);
@@ -1692,15 +1970,39 @@ hipError_t prefill_impl(const void* q, const void* k_cache, const void* v_cache,
     TileEntry* tiles = reinterpret_cast<TileEntry*>(ws + L.tiles_off);
     int32_t* dec = reinterpret_cast<int32_t*>(ws + L.dec_off);
     uint32_t* zero_row = reinterpret_cast<uint32_t*>(ws + L.zero_off);
+    // Small batches whose table rows are short enough run their single-token requests
+    // inside the tile launch (fused_dec): no decode launches at all, which a pure prompt
+    // batch -- most prefill steps -- would otherwise pay for work known on the device only.
+    const int Dk = decode_mfma_dim(head_dim);
+    const int64_t dec_groups = static_cast<int64_t>(batch_size) * num_kv_heads *
+                               dcore::decode_head_rep(num_q_heads / num_kv_heads);
+    const bool fused_dec = pipe_head_dim(Dk) && dec_groups <= kFusedDecodeGroups &&
+                           static_cast<int64_t>(max_blocks_per_req) * block_size <=
+                               kFusedDecodeMaxCtx;
+    const bool fork = !fused_dec && overlap != nullptr && overlap->side != nullptr &&
+                      batch_size >= kOverlapMinRequests;
+    // Beside decode items on a side stream the CUs are busy anyway: no split. Nor without the
+    // memory for it.
+    const size_t split_need = prefill_split_bytes(head_dim, max_blocks_per_req, block_size);
+    const bool can_split = L.split && !fork && split_need > 0 && split_bytes >= split_need;
+    char* sws = reinterpret_cast<char*>(align256(reinterpret_cast<uintptr_t>(split_ws)));
+    SplitTile* split = reinterpret_cast<SplitTile*>(sws);
+    SplitEntry* entries = reinterpret_cast<SplitEntry*>(split + kSplitCus / 2);
+    float* part_o = reinterpret_cast<float*>(sws + kSplitListBytes);
+    float* part_ml = part_o + kSplitRows * Dk;
+    SplitPlan sp{split, entries, can_split ? L.units : 0, L.gain,
+                 static_cast<int>(std::min<int64_t>(
+                     static_cast<int64_t>(max_blocks_per_req) * block_size, 0x7fffffff))};
     if (batch_size > kMaxPlanRequests) {
         int* big = reinterpret_cast<int*>(ws + L.big_off);
-        prefill_plan_kernel<true><<<1, 1024, 0, stream>>>(
+        prefill_plan_kernel<true, false><<<1, 1024, 0, stream>>>(
             query_start_loc, context_lens, batch_size, total_query_tokens, L.tile_tokens, counts,
-            tiles, dec, zero_row, decode_mfma_dim(head_dim) / 2, big, big + batch_size, 1);
+            tiles, dec, zero_row, decode_mfma_dim(head_dim) / 2, big, big + batch_size, 1, sp);
     } else {
-        prefill_plan_kernel<false><<<1, 1024, 0, stream>>>(
+        auto plan = sp.units > 0 ? prefill_plan_kernel<false, true> : prefill_plan_kernel<false, false>;
+        plan<<<1, 1024, 0, stream>>>(
             query_start_loc, context_lens, batch_size, total_query_tokens, L.tile_tokens, counts,
-            tiles, dec, zero_row, decode_mfma_dim(head_dim) / 2, nullptr, nullptr, 1);
+            tiles, dec, zero_row, decode_mfma_dim(head_dim) / 2, nullptr, nullptr, 1, sp);
     }
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
@@ -1729,17 +2031,6 @@ hipError_t prefill_impl(const void* q, const void* k_cache, const void* v_cache,
                                     items, max_blocks_per_req, num_q_heads, num_kv_heads,
                                     head_dim, block_size, L.plan, ws + L.decode_ws_off, s);
     };
-    // Small batches whose table rows are short enough run their single-token requests
-    // inside the tile launch (fused_dec): no decode launches at all, which a pure prompt
-    // batch -- most prefill steps -- would otherwise pay for work known on the device only.
-    const int Dk = decode_mfma_dim(head_dim);
-    const int64_t dec_groups = static_cast<int64_t>(batch_size) * num_kv_heads *
-                               dcore::decode_head_rep(num_q_heads / num_kv_heads);
-    const bool fused_dec = pipe_head_dim(Dk) && dec_groups <= kFusedDecodeGroups &&
-                           static_cast<int64_t>(max_blocks_per_req) * block_size <=
-                               kFusedDecodeMaxCtx;
-    const bool fork = !fused_dec && overlap != nullptr && overlap->side != nullptr &&
-                      batch_size >= kOverlapMinRequests;
     // Once the side stream has waited on the fork event it is joined back on every path,
     // errors included (an unjoined fork would invalidate a capture of the caller's stream).
     auto join = [&](hipError_t first) {
@@ -1765,7 +2056,7 @@ hipError_t prefill_impl(const void* q, const void* k_cache, const void* v_cache,
                              query_start_loc, context_lens, output, total_query_tokens,      \
                              max_blocks_per_req, num_q_heads, num_kv_heads, block_size,      \
                              counts, tiles, zero_row, L.max_tiles, stream, head_dim,         \
-                             batch_size, fused_dec)
+                             batch_size, fused_dec, sp, part_o, part_ml)
     if (F8 && pad) {
         err = hipErrorInvalidValue;  // fp8 runs the native head dims only
     } else {
@@ -1794,11 +2085,13 @@ hipError_t prefill_attention(const void* q, const void* k_cache, const void* v_c
                              const int32_t* context_lens, void* output, int batch_size,
                              int total_query_tokens, int max_blocks_per_req, int num_q_heads,
                              int num_kv_heads, int head_dim, int block_size, void* workspace,
-                             hipStream_t stream, const PrefillOverlap* overlap) {
+                             void* split_ws, size_t split_bytes, hipStream_t stream,
+                             const PrefillOverlap* overlap) {
     return prefill_impl<false>(q, k_cache, v_cache, nullptr, nullptr, block_table,
                                query_start_loc, context_lens, output, batch_size,
                                total_query_tokens, max_blocks_per_req, num_q_heads, num_kv_heads,
-                               head_dim, block_size, workspace, stream, overlap);
+                               head_dim, block_size, workspace, split_ws, split_bytes, stream,
+                               overlap);
 }
 
 // ---- any-layout prefill (the tile kernel with kAny) ----
@@ -1821,7 +2114,7 @@ AnyLayout any_layout(int batch_size, int total_query_tokens, int num_q_heads, in
     L.max_tiles = total_query_tokens / L.tile_tokens + batch_size;
     size_t off = 0;
     L.counts_off = off;
-    off = align256(off + 2 * sizeof(int32_t));
+    off = align256(off + 3 * sizeof(int32_t));
     L.tiles_off = off;
     off = align256(off + static_cast<size_t>(L.max_tiles) * sizeof(TileEntry));
     L.dec_off = off;
@@ -1859,16 +2152,17 @@ hipError_t prefill_attention_any(const void* q, const void* k_cache, const void*
     int32_t* counts = reinterpret_cast<int32_t*>(ws + L.counts_off);
     TileEntry* tiles = reinterpret_cast<TileEntry*>(ws + L.tiles_off);
     int32_t* dec = reinterpret_cast<int32_t*>(ws + L.dec_off);
+    const SplitPlan whole{nullptr, nullptr, 0, 0, 0x7fffffff};
     // single-token requests run as one-row tiles (the decode kernels take 16-token blocks)
     if (batch_size > kMaxPlanRequests) {
         int* big = reinterpret_cast<int*>(ws + L.big_off);
-        prefill_plan_kernel<true><<<1, 1024, 0, stream>>>(
+        prefill_plan_kernel<true, false><<<1, 1024, 0, stream>>>(
             query_start_loc, context_lens, batch_size, total_query_tokens, L.tile_tokens, counts,
-            tiles, dec, nullptr, 0, big, big + batch_size, 0);
+            tiles, dec, nullptr, 0, big, big + batch_size, 0, whole);
     } else {
-        prefill_plan_kernel<false><<<1, 1024, 0, stream>>>(
+        prefill_plan_kernel<false, false><<<1, 1024, 0, stream>>>(
             query_start_loc, context_lens, batch_size, total_query_tokens, L.tile_tokens, counts,
-            tiles, dec, nullptr, 0, nullptr, nullptr, 0);
+            tiles, dec, nullptr, 0, nullptr, nullptr, 0, whole);
     }
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
@@ -1897,13 +2191,14 @@ hipError_t prefill_attention_fp8(const void* q, const void* k_cache, const void*
                                  const int32_t* context_lens, void* output, int batch_size,
                                  int total_query_tokens, int max_blocks_per_req,
                                  int num_q_heads, int num_kv_heads, int head_dim,
-                                 void* workspace, hipStream_t stream,
-                                 const PrefillOverlap* overlap) {
+                                 void* workspace, void* split_ws, size_t split_bytes,
+                                 hipStream_t stream, const PrefillOverlap* overlap) {
     if (!pipe_head_dim(head_dim)) return hipErrorInvalidValue;
     return prefill_impl<true>(q, k_cache, v_cache, k_scale, v_scale, block_table,
                               query_start_loc, context_lens, output, batch_size,
                               total_query_tokens, max_blocks_per_req, num_q_heads, num_kv_heads,
-                              head_dim, kBlock, workspace, stream, overlap);
+                              head_dim, kBlock, workspace, split_ws, split_bytes, stream,
+                              overlap);
 }
 
 }  // namespace ccinfer::hipk

@@ -215,7 +215,7 @@ def _workspace(nbytes: int, device, workspace: Optional[torch.Tensor]):
         _require(workspace.is_cuda and workspace.numel() * workspace.element_size() >= nbytes,
                  "workspace")
         return workspace, workspace.numel() * workspace.element_size()
-    return torch.zeros(nbytes, dtype=torch.uint8, device=device), nbytes
+    return torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes
 
 
 def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,

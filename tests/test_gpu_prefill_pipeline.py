@@ -12,7 +12,7 @@ import pytest
 import torch
 
 import oracle
-from ccinfer_amd import prefill_attention, prefill_attention_fp8
+from ccinfer_amd import _lib, prefill_attention, prefill_attention_fp8, prefill_workspace_size
 from ccinfer_amd import workloads as W
 from tests._util import assert_attn_close, f32, say, u16
 from tests.test_gpu_fp8 import quantised_cache
@@ -90,3 +90,62 @@ def test_fp8_edges(gpu, d, hq, hkv, kind):
                                   vs.cpu().numpy(), w.block_table, w.query_start_loc,
                                   w.context_lens)
         assert_attn_close(f32(out), want, f"prefix {prefix}")
+
+
+# Launches that fill at most half the CUs split their tiles' key ranges (prefill_attn.hip, "Split
+# tiles"): prefix, new tokens of each request, query heads, kv heads, head dim.
+SPLIT = [
+    (1136, (17,), 16, 8, 128),
+    (1984, (512,), 16, 8, 128),
+    (3008, (64, 1, 200), 32, 8, 128),
+    (9008, (40, 1), 4, 4, 64),
+    (4000, (257, 100), 8, 2, 64),
+    (2992, (129,), 8, 2, 96),
+    (1200, (2, 3, 1, 5, 6), 1, 1, 128),
+    (0, (1600,), 4, 2, 128),
+]
+
+
+@pytest.mark.parametrize("holes", [False, True])
+@pytest.mark.parametrize("prefix,news,hq,hkv,d", SPLIT)
+def test_split_tiles(gpu, prefix, news, hq, hkv, d, holes):
+    say(f"split prefill prefix={prefix} new={news} {hq}/{hkv} d={d} holes={holes}")
+    w = W.prefill_prefix(device=gpu, seed=prefix + d, n_seqs=len(news), prefix=prefix, new=news,
+                         share_pairs=(), hq=hq, hkv=hkv, d=d)
+    _ramp(w, "grow")
+    if holes:
+        w.block_table[0, 3:9] = -1
+        w.block_table[-1, w.block_table.shape[1] // 2 + 1] = -1
+    m = w.device_meta(gpu)
+    size = prefill_workspace_size(w.batch, int(w.query_start_loc[-1]), w.mbpr, hq, hkv, d)
+    outs = []
+    for fill in (0xFF, 0x3C):  # the workspace needs no initialisation
+        ws = torch.full((size,), fill, dtype=torch.uint8, device=gpu)
+        outs.append(prefill_attention(w.q, w.k_cache, w.v_cache, m["block_table"],
+                                      m["query_start_loc"], m["context_lens"], workspace=ws))
+    # a workspace without room for the partials (the size also holds two copies of the q rows)
+    rows = 2 * (-(-w.q.numel() * 2 // 256) * 256)
+    ws = torch.empty(size - rows - (1 << 20), dtype=torch.uint8, device=gpu)
+    whole = torch.empty_like(w.q)
+    code = _lib.load().ccinfer_prefill_attention(
+        *(x.data_ptr() for x in (w.q, w.k_cache, w.v_cache, m["block_table"], m["query_start_loc"],
+                                 m["context_lens"], whole)),
+        w.batch, w.q.shape[0], w.mbpr, hq, hkv, d, 16, ws.data_ptr(), ws.numel(),
+        torch.cuda.current_stream().cuda_stream)
+    assert code == 0
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    want = oracle.prefill(u16(w.q), u16(w.k_cache), u16(w.v_cache), w.block_table,
+                          w.query_start_loc, w.context_lens)
+    assert_attn_close(f32(outs[0]), want, "split")
+    assert_attn_close(f32(whole), want, "whole")
+    assert not torch.equal(outs[0], whole)  # the batch did split
+    if not holes and d in (64, 128):
+        kc, vc, ks, vs = quantised_cache(gpu, w, hkv, d)
+        o8 = prefill_attention_fp8(w.q, kc, vc, ks, vs, m["block_table"], m["query_start_loc"],
+                                   m["context_lens"])
+        torch.cuda.synchronize()
+        want = oracle.prefill_fp8(u16(w.q), kc.cpu().numpy(), vc.cpu().numpy(), ks.cpu().numpy(),
+                                  vs.cpu().numpy(), w.block_table, w.query_start_loc,
+                                  w.context_lens)
+        assert_attn_close(f32(o8), want, "split fp8")
