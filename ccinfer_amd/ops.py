@@ -21,6 +21,7 @@ allocator unless passed in (scratch: no initialisation needed).
 """
 from __future__ import annotations
 
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -44,6 +45,12 @@ def _check(code: int, op: str) -> None:
         raise CcinferError(code, op)
 
 
+# The smallest decode call takes 8 us on the GPU, so its host side bounds it: the checks below
+# are written for few interpreter steps, the stream handle is read without building a
+# torch.cuda.Stream, and size queries (pure functions of their whole-number arguments; typed, so
+# that a value ctypes refuses is refused again) are remembered. Host time of a call, before and
+# after: decode_attention 12.2 -> 8.7 us, prefill_attention with its write 26.4 -> 20.3 us.
+
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
@@ -54,11 +61,13 @@ def _require(cond: bool, op: str) -> None:
 
 
 def _dev_tensor(t: Optional[torch.Tensor], dtype: torch.dtype, op: str) -> None:
-    _require(t is not None and t.is_cuda and t.dtype == dtype and t.is_contiguous(), op)
+    if t is None or t.dtype is not dtype or not t.is_cuda or not t.is_contiguous():
+        raise CcinferError(INVALID_ARGUMENT, op)
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The raw handle of torch's current stream (torch.cuda.current_stream().cuda_stream)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 class SideStream:
@@ -194,12 +203,14 @@ def build_batch_metadata(item_kv_written: torch.Tensor, item_new_tokens: torch.T
     return out
 
 
+@lru_cache(maxsize=1024, typed=True)
 def decode_workspace_size(batch_size: int, max_blocks_per_req: int, num_q_heads: int,
                           num_kv_heads: int, head_dim: int, cache_block_size: int = 16) -> int:
     return int(_lib.load().ccinfer_decode_workspace_size(
         batch_size, max_blocks_per_req, num_q_heads, num_kv_heads, head_dim, cache_block_size))
 
 
+@lru_cache(maxsize=1024, typed=True)
 def prefill_workspace_size(batch_size: int, total_query_tokens: int, max_blocks_per_req: int,
                            num_q_heads: int, num_kv_heads: int, head_dim: int,
                            cache_block_size: int = 16) -> int:
@@ -212,9 +223,9 @@ def _workspace(nbytes: int, device, workspace: Optional[torch.Tensor]):
     if nbytes == 0:
         return None, 0
     if workspace is not None:
-        _require(workspace.is_cuda and workspace.numel() * workspace.element_size() >= nbytes,
-                 "workspace")
-        return workspace, workspace.numel() * workspace.element_size()
+        have = workspace.numel() * workspace.element_size()
+        _require(workspace.is_cuda and have >= nbytes, "workspace")
+        return workspace, have
     return torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes
 
 
@@ -245,6 +256,7 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     return output
 
 
+@lru_cache(maxsize=1024, typed=True)
 def decode_shared_workspace_size(batch_size: int, max_blocks_per_req: int, num_q_heads: int,
                                  num_kv_heads: int, head_dim: int,
                                  cache_block_size: int = 16) -> int:
