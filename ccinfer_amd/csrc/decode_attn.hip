@@ -590,25 +590,52 @@ __device__ void merge_row_two(const float* __restrict__ ws_o, const float* __res
 // prefix is read once per subgroup instead of once per request. Each member's positions from
 // the end of the prefix on run through the ordinary split plan (items start there), and the
 // merge adds the prefix partials to the row. Requests in no group run as in plain decode.
-constexpr int kSharedSplitTokens = 128;   // prefix positions per shared-kernel wavefront
+constexpr int kSharedSplitTokens = 128;   // workspace: partial slots per this many positions
+constexpr int kSharedMinPiece = 64;       // smallest and largest prefix piece of a wavefront
+constexpr int kSharedMaxPiece = 2048;     // (largest: 64 lanes hold 2 block ids each)
+constexpr int kSharedPiece = 256;         // its length where that fits the wavefronts,
+constexpr int kSharedSpread = 4;          // or shorter until 1 / 4 of them have one
 constexpr int kSharedMinTokens = 64;      // shorter common prefixes are not worth a subgroup
 constexpr int kSharedMaxItems = 2048;     // the planner's hash table holds 2x this many keys
 constexpr int kSharedHash = 4096;
 constexpr int kSharedCols = 16;           // columns of the 16x16x32 MFMA tile
-constexpr int kSharedSlotsPerHead = 128;  // shared-kernel wavefronts per kv head
+constexpr int kSharedWaves = 2048;        // shared-kernel wavefronts, all resident at D = 128
 
 struct SharedPlan {
     int32_t* nsub;      // [1] subgroups
     int32_t* sub_len;   // [B] prefix positions of subgroup s
-    int32_t* sub_n;     // [B] members of subgroup s
+    int32_t* sub_n;     // [B] members of subgroup s, and above bit 8 the positions per piece
     int32_t* sub_mem;   // [B][16] its members (items)
     int32_t* begin;     // [B] first position item r attends in the split plan
     int32_t* sh_splits; // [B] prefix partials of item r's rows
+    int32_t* pieces;    // [1] most pieces of any subgroup
 };
+
+// Prefix positions per piece of a subgroup's prefix of len positions, where nsub subgroups
+// share `slots` wavefronts per kv head: at most one piece per wavefront. A long piece costs
+// its own latency; a short one costs a partial row of every member (written here, read by the
+// merge) and contends with the split work, which runs beside. With 128 positions always (and
+// few items crowded on the first XCDs) against this rule, us a call, D = 128:
+//   64 requests, prefix 2,048 (Hq/Hkv 16/8)       61.5 -> 58.9
+//   100 requests, two prefixes of 4,096 (32/8)   128.9 -> 97.6
+//   256 requests, two of 1,024 (16/8)             92.0 -> 87.0
+//   4 requests, 8,000 (32/8)                      40.0 -> 35.1
+//   64 requests, 2,048 (16/2; 32/32)              54.9 -> 39.7; 80.1 -> 61.9
+//   8 requests, 512 (16/8)                        21.3 -> 19.3
+// Also tried: kSharedPiece 384 and 512 (256 requests: 102.6), smallest piece 96 or 128
+// (8 requests: 20.4, 21.4), 1,024 wavefronts (100 requests: 102.5), pieces chosen by rounds
+// times length (no better, and its loop costs the planner 0.7).
+__device__ __forceinline__ int shared_piece(int len, int nsub, int slots, int sh_k) {
+    const int lo = (len - 1) / kSharedMaxPiece + 1;
+    const int hi = max(lo, min(sh_k, len / kSharedMinPiece));
+    const int most = slots / nsub;
+    const int n = min(max(max(min(len / kSharedPiece, most), most / kSharedSpread), lo), hi);
+    return ((len - 1) / n / kChunk + 1) * kChunk;
+}
 
 __global__ __launch_bounds__(1024) void decode_shared_plan_kernel(
     const int32_t* __restrict__ block_table, const int32_t* __restrict__ context_lens, int B,
-    int mbpr, int M, SharedPlan sp) {
+    int mbpr, int M, int slots, int sh_k, SharedPlan sp) {
     __shared__ int h_key[kSharedHash];
     __shared__ int h_lead[kSharedHash];
     __shared__ int h_count[kSharedHash];
@@ -617,6 +644,7 @@ __global__ __launch_bounds__(1024) void decode_shared_plan_kernel(
     __shared__ int h_base[kSharedHash];
     __shared__ int h_slot[kSharedMaxItems];  // each request's hash slot (-1: not grouped)
     __shared__ int s_nsub;
+    __shared__ int s_pieces;
     constexpr int kPer = kSharedMaxItems / 1024;
     const int tid = threadIdx.x;
     for (int i = tid; i < kSharedHash; i += 1024) {
@@ -627,7 +655,7 @@ __global__ __launch_bounds__(1024) void decode_shared_plan_kernel(
         h_common[i] = 0x7fffffff;
         h_base[i] = 0;  // the fill counter until the subgroups are numbered
     }
-    if (tid == 0) s_nsub = 0;
+    if (tid == 0) s_nsub = s_pieces = 0;
     __syncthreads();
     // 1. hash every eligible request on its first block id (decode semantics: a row whose
     //    context is invalid writes zeros and is never grouped)
@@ -740,17 +768,24 @@ __global__ __launch_bounds__(1024) void decode_shared_plan_kernel(
         const int len = h_common[h];
         sp.sub_mem[sub * kSharedCols + i % M] = r;
         sp.begin[r] = len;
-        sp.sh_splits[r] = (len + kSharedSplitTokens - 1) / kSharedSplitTokens;
+        const int piece = shared_piece(len, s_nsub, slots, sh_k);
+        const int pieces = (len - 1) / piece + 1;
+        sp.sh_splits[r] = pieces;
         if (i % M == 0) {
             sp.sub_len[sub] = len;
-            sp.sub_n[sub] = min(M, h_count[h] - (i / M) * M);
+            atomicMax(&s_pieces, pieces);
+            sp.sub_n[sub] = min(M, h_count[h] - (i / M) * M) | piece << 8;
         }
     }
-    if (tid == 0) *sp.nsub = s_nsub;
+    __syncthreads();
+    if (tid == 0) {
+        *sp.nsub = s_nsub;
+        *sp.pieces = s_pieces;
+    }
 }
 
-// Prefix attention of the subgroups: each wavefront takes work items (128-position piece,
-// kv head h, subgroup) in turn. Lane column j holds
+// Prefix attention of the subgroups: each wavefront takes work items (piece, kv head h,
+// subgroup) in turn. Lane column j holds
 // member j / G's query head h G + j % G; the partial (O, m, l) of each member row goes to
 // the shared area at ((member * Hq + head) * k + piece).
 // Runs in the split kernel's extra workgroups (wg of nwg), beside the split work, which
@@ -768,24 +803,28 @@ __device__ __forceinline__ void shared_prefix_work(
     // Work item (piece, kv head, subgroup), subgroup fastest: the wavefronts of a workgroup
     // read the same K/V rows (they hit in the CU's cache), and workgroups are renumbered so
     // that consecutive ones run on one XCD (workgroups are dealt to the 8 XCDs in turn),
-    // keeping the subgroups of a piece in one L2.
+    // keeping the subgroups of a piece in one L2. Fewer items than wavefronts are spread over
+    // all XCDs: the workgroups that would have none leave first.
     // nwg: a multiple of 8; the split workgroups before these are a multiple of 8 too
-    const int wg = (wg_raw % 8) * (nwg / 8) + wg_raw / 8;
+    const int nsub = *sp.nsub;
+    const int nwork = nsub * hkv * *sp.pieces;
+    const int used = min(nwg, (nwork + 8 * kWavesPerGroup - 1) / (8 * kWavesPerGroup) * 8);
+    if (wg_raw >= used) return;
+    const int wg = (wg_raw % 8) * (used / 8) + wg_raw / 8;
     const int wi = wg * kWavesPerGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int G = hq / hkv;
     const int j = lane & 15;
     const int g = lane >> 4;
-    const int nsub = *sp.nsub;
-    const int nwork = nsub * hkv * sh_k;
-    for (int w = wi; w < nwork; w += nwg * kWavesPerGroup) {
+    for (int w = wi; w < nwork; w += used * kWavesPerGroup) {
         const int sub = w % nsub;
         const int h = (w / nsub) % hkv;
         const int piece = w / (nsub * hkv);
         const int len = sp.sub_len[sub];
-        const int begin = piece * kSharedSplitTokens;
+        const int shape = sp.sub_n[sub];
+        const int nmem = shape & 0xff;
+        const int begin = piece * (shape >> 8);
         if (begin >= len) continue;  // wave-uniform
-        const int end = min(len, begin + kSharedSplitTokens);
-        const int nmem = sp.sub_n[sub];
+        const int end = min(len, begin + (shape >> 8));
         const int32_t* mem = sp.sub_mem + sub * kSharedCols;
         const int m = j / G;
         const bool live = m < nmem;
@@ -1464,14 +1503,16 @@ hipError_t launch_decode_shared(const void* q, const void* k_cache, const void* 
     sp.begin = sp.sub_n + B;
     sp.sh_splits = sp.begin + B;
     sp.sub_mem = sp.sh_splits + B;
+    sp.pieces = sp.sub_mem + B * kSharedCols;
     float* sh_o = reinterpret_cast<float*>(ws + L.o_off);
     float* sh_ml = reinterpret_cast<float*>(ws + L.ml_off);
     const int G = hq / hkv;
+    const int slots = std::max(1, kSharedWaves / hkv);  // wavefronts per kv head
     decode_shared_plan_kernel<<<1, 1024, 0, stream>>>(block_table, context_lens, B, mbpr,
-                                                      kSharedCols / G, sp);
+                                                      kSharedCols / G, slots, L.k, sp);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
-    const int waves = kSharedSlotsPerHead * hkv;
+    const int waves = slots * hkv;
     const int nwg = ((waves + kWavesPerGroup - 1) / kWavesPerGroup + 7) / 8 * 8;
     ItemArgs it{};
     it.num_items = B;

@@ -116,3 +116,20 @@ def test_repeatable(gpu):
     first = run(decode_attention_shared_prefix, w, gpu).clone()
     for _ in range(3):
         assert torch.equal(run(decode_attention_shared_prefix, w, gpu), first)
+
+
+@pytest.mark.parametrize("batch,prefix,groups,hq,hkv,d", [
+    (2, 64, 1, 16, 8, 128),       # the shortest prefix: one piece
+    (9, 160, 1, 16, 8, 128),      # a piece of 96 and a ragged one of 64
+    (2, 30000, 1, 8, 2, 128),     # over a hundred pieces a row: the merge's second round
+    (5, 2080, 2, 16, 2, 64),      # pieces cut to the workspace's slots per row
+    (66, 2080, 1, 512, 64, 32),   # more subgroups than wavefronts per head: two long pieces
+])
+def test_prefix_pieces(gpu, batch, prefix, groups, hq, hkv, d):
+    """The piece length's rule at its limits; the bar is this file's."""
+    say(f"prefix pieces b={batch} prefix={prefix} groups={groups} hq={hq} hkv={hkv} d={d}")
+    w = W.decode_shared_prefix(device=gpu, seed=batch + prefix, batch=batch, prefix=prefix,
+                               priv_lo=1, priv_hi=60, groups=groups, hq=hq, hkv=hkv, d=d)
+    poison_unused(w, gpu)
+    got = f32(run(decode_attention_shared_prefix, w, gpu))
+    assert_attn_close(got, oracle_decode(w), w.name)
