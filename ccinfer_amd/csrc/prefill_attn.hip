@@ -903,10 +903,10 @@ struct PipeShape {
 
 __host__ __device__ constexpr bool pipe_head_dim(int d) { return d == 64 || d == 128; }
 
-// F8: the cache holds OCP E4M3 bytes with row scales (k_scale / v_scale). Tiles are then
-// staged as bytes into a two-tile ring and dequantised (byte * row scale, rounded to bf16)
-// into a two-tile ring of bf16 tiles in the same swizzled layout, so everything after the
-// staging is the bf16 kernel.
+// F8: the cache holds OCP E4M3 bytes with row scales (k_scale / v_scale). A tile's bytes are
+// then loaded into registers and dequantised (byte * row scale, rounded to bf16) into the same
+// rings of bf16 tiles in the same swizzled layout, so everything after the staging is the bf16
+// kernel.
 // kPad (bf16 only): q / cache / output rows hold dr < D dims (a multiple of 8). Staging
 // fetches chunk 0 of the row again in place of the missing chunks (finite values: the Q
 // operand is zero in those dims, so they add exactly 0 to the scores), and the missing
@@ -1297,7 +1297,7 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     // In half-step h (half h % 2 of tile h / 2) a wavefront runs, none depending on another:
     //     S(h + 2) = K . Q^T         (S2 MFMAs, one accumulator chain)
     //     O += V(h)^T . P(h)^T       (S2 MFMAs, NT2 chains)
-    //     P(h + 1) = exp2(S(h + 1) * scale - m), after the row max of S(h + 1)
+    //     P(h + 1) = exp2(S(h + 1) * scale - m), its row max only where a row outgrew m
     // so its instruction stream alternates a QK and a PV MFMA with a quarter of the VALU
     // work's share between each two, and every operand is read from LDS two MFMAs of its kind
     // ahead. The order is pinned slot by slot (sched_barrier): left to the scheduler's
