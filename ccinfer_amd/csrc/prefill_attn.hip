@@ -1247,7 +1247,7 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
         const __bf16* qv = q + (static_cast<int64_t>(qb + (live ? tq : 0)) * hq + q_head) * ds;
 #pragma unroll
         for (int kk = 0; kk < S2; ++kk) {
-            // rows past the tile's end read row 0 (finite) and are never stored
+            // rows past the tile's end read the request's first row and are never stored
             const bool ok = !kPad || kk * 16 + h32 * 8 < dr;
             u32x4 w = load16(qv + (ok ? kk * 16 + h32 * 8 : 0));
             if (!ok) w = u32x4{0, 0, 0, 0};
@@ -1376,6 +1376,33 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
         p[0] = __builtin_bit_cast(bf16x8, w[0]);
         p[1] = __builtin_bit_cast(bf16x8, w[1]);
     };
+    // Whether a P word holds a probability of 2 or more, or one that is not finite: bit 14 of a
+    // bf16.
+    auto reaches_two = [](const u32x4& w0, const u32x4& w1) __attribute__((always_inline)) {
+        const uint32_t bits = (w0[0] | w0[1] | w0[2]) | (w0[3] | w1[0] | w1[1]) | (w1[2] | w1[3]);
+        return __builtin_amdgcn_ballot_w64((bits & 0x40004000u) != 0);
+    };
+    // The row sums put two query rows in one MFMA column, where a NaN or Inf of one would reach
+    // the other (0 * NaN). So after exp_all with a reference kRefHead above each row's max, when
+    // a P that still reaches two is not finite (a query row, or a score of it, was not): such
+    // rows, in both lanes that hold them, continue with P = 0 and the NaN kept in acc. The bits
+    // are set by integer operations, since the build lets the compiler assume there are no NaNs.
+    auto settle = [&](bf16x8 (&p)[2]) __attribute__((always_inline)) {
+        u32x4 w[2] = {__builtin_bit_cast(u32x4, p[0]), __builtin_bit_cast(u32x4, p[1])};
+        const uint64_t lanes = reaches_two(w[0], w[1]);
+        if (__builtin_expect(lanes != 0, 0)) {
+            const bool bad = ((lanes | lanes >> 32 | lanes << 32) >> lane & 1) != 0;
+            const uint32_t nan = bad ? 0x7fc00000u : 0u;
+            const uint32_t keep = bad ? 0u : 0xffffffffu;
+#pragma unroll
+            for (int n = 0; n < NT2; ++n)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    acc[n][v] = __uint_as_float(__float_as_uint(acc[n][v]) | nan);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) p[s] = __builtin_bit_cast(bf16x8, w[s] & keep);
+        }
+    };
     bf16x8 kop[4], vop[4];  // operands read ahead (two of each kind) and the one in use
 
     // One half-step, hh = h % 2. kQk: sq = S of half hh of the K tile (kMask: from the seed in
@@ -1450,13 +1477,12 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
         if constexpr (kExp) {
             pe[0] = __builtin_bit_cast(bf16x8, pw[0]);
             pe[1] = __builtin_bit_cast(bf16x8, pw[1]);
-            const uint32_t bits = (pw[0][0] | pw[0][1] | pw[0][2]) | (pw[0][3] | pw[1][0] | pw[1][1]) |
-                                  (pw[1][2] | pw[1][3]);
-            if (__builtin_amdgcn_ballot_w64((bits & 0x40004000u) != 0) != 0) {
+            if (reaches_two(pw[0], pw[1]) != 0) {
                 const float m_new = fmaxf(m, row_ref(se));
                 rescale(__builtin_amdgcn_exp2f(m - m_new));
                 m = m_new;
                 exp_all(se, pe);
+                settle(pe);
             }
         }
     };
@@ -1545,6 +1571,7 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
             }
             m = fmaxf(m, row_ref(s_even));
             exp_all(s_even, p_even);
+            settle(p_even);
         }
         // Byte offsets of the ring slots: step t reads K of tile t + 1 and V of tile t.
         int slot = 0;  // kTileBytes * ((t - kt0) % 3)

@@ -1,0 +1,66 @@
+"""Prefill with non-finite values: what a NaN or Inf may reach in the pipelined kernel.
+
+Every query row attends by itself (src/kernel/attention/prefill_attn.cu:80-241: one row's
+running max, sum and accumulator), so a NaN or Inf in one query row leaves every other row as
+it is without it. The comparison is with the same call without the bad row, at the suite's bar:
+wavefronts move the references of their rows together, which changes roundings only.
+"""
+import pytest
+import torch
+
+from ccinfer_amd import prefill_attention, prefill_attention_fp8
+from ccinfer_amd import workloads as W
+from tests._util import assert_attn_close, f32, say
+from tests.test_gpu_fp8 import quantised_cache
+
+pytestmark = pytest.mark.gpu
+
+NAN, INF = float("nan"), float("inf")
+
+# prefix, new tokens of each request, query heads, kv heads, head dim
+WHOLE = [
+    (0, (10, 16, 17), 16, 8, 128),       # partial tiles: rows past the end repeat the first row
+    (48, (40, 200), 3, 3, 128),
+    (0, (130, 33), 32, 8, 64),
+    (16, (70, 100), 4, 2, 96),           # padded head dim
+]
+SPLIT = [
+    (1984, (512,), 16, 8, 128),
+    (3008, (20, 200), 32, 8, 128),
+    (4000, (257,), 8, 2, 64),
+]
+
+
+def _inputs(gpu, prefix, news, hq, hkv, d):
+    return W.prefill_prefix(device=gpu, seed=prefix + d, n_seqs=len(news), prefix=prefix, new=news,
+                            share_pairs=(), hq=hq, hkv=hkv, d=d)
+
+
+def _calls(gpu, w, hkv, d):
+    """The bf16 call and, where it exists, the fp8 call, as functions of q."""
+    m = w.device_meta(gpu)
+    meta = (m["block_table"], m["query_start_loc"], m["context_lens"])
+    yield "bf16", lambda q: prefill_attention(q, w.k_cache, w.v_cache, *meta)
+    if d in (64, 128):
+        kc, vc, ks, vs = quantised_cache(gpu, w, hkv, d)
+        yield "fp8", lambda q: prefill_attention_fp8(q, kc, vc, ks, vs, *meta)
+
+
+@pytest.mark.parametrize("bad", [NAN, INF])
+@pytest.mark.parametrize("prefix,news,hq,hkv,d", WHOLE + SPLIT)
+def test_query_rows_are_independent(gpu, prefix, news, hq, hkv, d, bad):
+    w = _inputs(gpu, prefix, news, hq, hkv, d)
+    starts = [int(x) for x in w.query_start_loc]
+    for kind, call in _calls(gpu, w, hkv, d):
+        want = f32(call(w.q))
+        for b, n in enumerate(news):
+            for r in sorted({0, 5, n // 2, n - 1}):
+                row, head = starts[b] + r, (r + b) % hq
+                say(f"bad query row {kind} {bad} {hq}/{hkv} d={d} prefix={prefix} new={n} row={r}")
+                q = w.q.clone()
+                q[row, head] = bad
+                got = f32(call(q))
+                if bad != bad:
+                    assert (got[row, head] != got[row, head]).all()
+                got[row, head] = want[row, head]
+                assert_attn_close(got, want, f"{kind}, bad row {r} of {n}")
