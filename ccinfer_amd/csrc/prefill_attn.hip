@@ -1477,7 +1477,7 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
         if constexpr (kExp) {
             pe[0] = __builtin_bit_cast(bf16x8, pw[0]);
             pe[1] = __builtin_bit_cast(bf16x8, pw[1]);
-            if (reaches_two(pw[0], pw[1]) != 0) {
+            if (__builtin_expect(reaches_two(pw[0], pw[1]) != 0, 0)) {
                 const float m_new = fmaxf(m, row_ref(se));
                 rescale(__builtin_amdgcn_exp2f(m - m_new));
                 m = m_new;
@@ -1561,7 +1561,12 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
                 __builtin_amdgcn_s_waitcnt(0x0F70);
         }
         __syncthreads();
-        {
+        // The key tiles of this wavefront: those after them lie wholly above its last row, and it
+        // only stages them (0 * V must not be formed there, since V may hold Inf or NaN). A piece
+        // of a split tile may have none at all: it then leaves m = kMaxInit and sums of 0.
+        const int wave_lim = prefix + tw + kPipeRows - 1;
+        const int wave_end = min(ntiles, wave_lim / kKeysPerTile + 1);
+        if (kt0 < wave_end) {
             mask_seed(s_even, kt0 * kKeysPerTile, valid_buf(kt0), 0, holes_tag);
             mask_seed(s_odd, kt0 * kKeysPerTile + 32, valid_buf(kt0), 1, holes_tag);
 #pragma unroll
@@ -1646,28 +1651,39 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
                     if (s == 3) fetch8_v(t + 3);
                 }
             };
+            // Half 1 of the last tile may lie wholly above the last row too: P = 0, and no PV.
+            const bool above = kLast && t * kKeysPerTile + 32 > wave_lim;
+            if (above) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) s_odd[v] = kNegInf;
+            }
             half_step(H0{}, s_even, s_odd, p_odd, p_even, turn, stage, Qk{}, T{}, Seed{}, T{});
             if constexpr (!F8 && !kMask) {
 #pragma unroll
                 for (int x = 0; x < NL; ++x) v_ids[x] = k_ids[x];
             }
             if constexpr (Seed::value) mask_seed(s_odd, key1 + 32, valid_buf(t + 1), 1, holes_tag);
-            half_step(H1{}, s_odd, s_even, p_even, p_odd, turn, stage1, Qk{}, Qk{}, Seed{}, Qk{});
+            if (!above) {
+                half_step(H1{}, s_odd, s_even, p_even, p_odd, turn, stage1, Qk{}, Qk{}, Seed{},
+                          Qk{});
+            } else {
+                stage1(1);
+                stage1(3);
+            }
             slot = next_slot(slot);
         };
-        // This wavefront's last tile: the ones after it lie wholly above its last row, and it
-        // only stages them.
-        const int wave_last =
-            max(kt0, min(ntiles - 1, (prefix + tw + kPipeRows - 1) / kKeysPerTile));
         int t = kt0;
         // Steps whose QK tile lies wholly below the workgroup's first query row need no mask.
         const int mask_free_tiles = (prefix + t0 + 1) / kKeysPerTile;
         const int fast_steps = kHoles ? 0 : min(mask_free_tiles - 1, full_tiles - 3);
-        if constexpr (!kHoles)
-            for (; t < fast_steps; ++t) step(t, F{}, F{});
-        for (; t < wave_last; ++t) step(t, T{}, F{});
-        step(t, T{}, T{});
-        for (++t; t < ntiles; ++t) {
+        if (kt0 < wave_end) {
+            if constexpr (!kHoles)
+                for (; t < fast_steps; ++t) step(t, F{}, F{});
+            for (; t < wave_end - 1; ++t) step(t, T{}, F{});
+            step(t, T{}, T{});
+            ++t;
+        }
+        for (; t < ntiles; ++t) {
             advance(t, F{});
             if constexpr (F8) {
                 if (t + 3 < ntiles) convert8(k8, slot);

@@ -4,6 +4,10 @@ Every query row attends by itself (src/kernel/attention/prefill_attn.cu:80-241: 
 running max, sum and accumulator), so a NaN or Inf in one query row leaves every other row as
 it is without it. The comparison is with the same call without the bad row, at the suite's bar:
 wavefronts move the references of their rows together, which changes roundings only.
+
+A key past a row's causal limit has probability 0 there, and 0 * NaN is NaN, so a non-finite
+cache row reaches earlier rows where the kernel multiplies it at all: in the 32-key half that
+holds the last key of the row's wavefront (32 query rows), never past it.
 """
 import pytest
 import torch
@@ -44,6 +48,43 @@ def _calls(gpu, w, hkv, d):
     if d in (64, 128):
         kc, vc, ks, vs = quantised_cache(gpu, w, hkv, d)
         yield "fp8", lambda q: prefill_attention_fp8(q, kc, vc, ks, vs, *meta)
+
+
+# prefix, new tokens, position of the bad cache row, query heads, kv heads, head dim: the rows of
+# wavefronts whose last key lies in an earlier 32-key half must not change a bit.
+LATER_KEYS = [
+    (0, 128, 40, 4, 2, 128),
+    (0, 128, 100, 4, 2, 128),
+    (16, 200, 150, 3, 3, 64),
+    (0, 64, 63, 4, 2, 96),
+    (1136, 256, 1391, 4, 4, 128),    # split: the last piece lies above the first wavefronts
+    (1136, 256, 1300, 4, 4, 128),
+    (4000, 256, 4255, 3, 3, 64),
+    (2992, 129, 3100, 8, 2, 96),
+]
+
+
+@pytest.mark.parametrize("prefix,new,pos,hq,hkv,d", LATER_KEYS)
+def test_rows_before_a_bad_cache_row(gpu, prefix, new, pos, hq, hkv, d):
+    w = _inputs(gpu, prefix, (new,), hq, hkv, d)
+    clean = [r for r in range(new) if (prefix + r // 32 * 32 + 31) // 32 < pos // 32]
+    assert 0 < len(clean) <= pos - prefix
+    slot = int(w.block_table[0, pos // 16]) * 16 + pos % 16
+    m = w.device_meta(gpu)
+    meta = (m["block_table"], m["query_start_loc"], m["context_lens"])
+    want = prefill_attention(w.q, w.k_cache, w.v_cache, *meta)
+    say(f"bad cache row prefix={prefix} new={new} pos={pos} {hq}/{hkv} d={d}")
+    for k, v in ((NAN, NAN), (1.0, INF), (INF, 1.0)):
+        kc, vc = w.k_cache.clone(), w.v_cache.clone()
+        kc[slot], vc[slot] = k, v
+        got = prefill_attention(w.q, kc, vc, *meta)
+        assert torch.equal(got[clean].view(torch.int16), want[clean].view(torch.int16)), (k, v)
+    if d in (64, 128):
+        kc, vc, ks, vs = quantised_cache(gpu, w, hkv, d)
+        want = prefill_attention_fp8(w.q, kc, vc, ks, vs, *meta)
+        kc[slot], vc[slot] = 0x7F, 0x7F  # E4M3 NaN
+        got = prefill_attention_fp8(w.q, kc, vc, ks, vs, *meta)
+        assert torch.equal(got[clean].view(torch.int16), want[clean].view(torch.int16)), "fp8"
 
 
 @pytest.mark.parametrize("bad", [NAN, INF])
