@@ -47,9 +47,9 @@ def _check(code: int, op: str) -> None:
 
 # The smallest decode call takes 8 us on the GPU, so its host side bounds it: the checks below
 # are written for few interpreter steps, the stream handle is read without building a
-# torch.cuda.Stream, and size queries (pure functions of their whole-number arguments; typed, so
-# that a value ctypes refuses is refused again) are remembered. Host time of a call, before and
-# after: decode_attention 12.2 -> 8.7 us, prefill_attention with its write 26.4 -> 20.3 us.
+# torch.cuda.Stream, and the sizes a call asks for are remembered (_size). Host time of a call,
+# before and after: decode_attention 12.2 -> 8.7 us, prefill_attention with its write 26.4 ->
+# 20.3 us.
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
@@ -203,20 +203,30 @@ def build_batch_metadata(item_kv_written: torch.Tensor, item_new_tokens: torch.T
     return out
 
 
-@lru_cache(maxsize=1024, typed=True)
 def decode_workspace_size(batch_size: int, max_blocks_per_req: int, num_q_heads: int,
                           num_kv_heads: int, head_dim: int, cache_block_size: int = 16) -> int:
     return int(_lib.load().ccinfer_decode_workspace_size(
         batch_size, max_blocks_per_req, num_q_heads, num_kv_heads, head_dim, cache_block_size))
 
 
-@lru_cache(maxsize=1024, typed=True)
 def prefill_workspace_size(batch_size: int, total_query_tokens: int, max_blocks_per_req: int,
                            num_q_heads: int, num_kv_heads: int, head_dim: int,
                            cache_block_size: int = 16) -> int:
     return int(_lib.load().ccinfer_prefill_workspace_size(
         batch_size, total_query_tokens, max_blocks_per_req, num_q_heads, num_kv_heads, head_dim,
         cache_block_size))
+
+
+@lru_cache(maxsize=1024)
+def _known_size(query, *args: int) -> int:
+    return query(*args)
+
+
+def _size(query, *args) -> int:
+    """A size query of a call's own shapes. They are plain ints of tensor shapes, except the last
+    argument, which is the caller's block size: it is looked up only where it is an int too (a
+    0-d tensor, which the query takes as well, compares by identity and may change its value)."""
+    return _known_size(query, *args) if type(args[-1]) is int else query(*args)
 
 
 def _workspace(nbytes: int, device, workspace: Optional[torch.Tensor]):
@@ -248,7 +258,7 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     _dev_tensor(output, torch.bfloat16, op)
     _require(output.shape == q.shape, op)
     mbpr = block_table.shape[1]
-    need = decode_workspace_size(b, mbpr, hq, hkv, d, cache_block_size)
+    need = _size(decode_workspace_size, b, mbpr, hq, hkv, d, cache_block_size)
     ws, ws_bytes = _workspace(need, q.device, workspace)
     _check(_lib.load().ccinfer_decode_attention(
         _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), _ptr(context_lens),
@@ -256,7 +266,6 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     return output
 
 
-@lru_cache(maxsize=1024, typed=True)
 def decode_shared_workspace_size(batch_size: int, max_blocks_per_req: int, num_q_heads: int,
                                  num_kv_heads: int, head_dim: int,
                                  cache_block_size: int = 16) -> int:
@@ -287,7 +296,7 @@ def decode_attention_shared_prefix(q: torch.Tensor, k_cache: torch.Tensor,
     _dev_tensor(output, torch.bfloat16, op)
     _require(output.shape == q.shape, op)
     mbpr = block_table.shape[1]
-    need = decode_shared_workspace_size(b, mbpr, hq, hkv, d, cache_block_size)
+    need = _size(decode_shared_workspace_size, b, mbpr, hq, hkv, d, cache_block_size)
     ws, ws_bytes = _workspace(need, q.device, workspace)
     _check(_lib.load().ccinfer_decode_attention_shared_prefix(
         _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), _ptr(context_lens),
@@ -320,7 +329,7 @@ def decode_attention_write_kv(q: torch.Tensor, k_new: torch.Tensor, v_new: torch
     _dev_tensor(output, torch.bfloat16, op)
     _require(output.shape == q.shape, op)
     mbpr = block_table.shape[1]
-    need = decode_workspace_size(b, mbpr, hq, hkv, d, cache_block_size)
+    need = _size(decode_workspace_size, b, mbpr, hq, hkv, d, cache_block_size)
     ws, ws_bytes = _workspace(need, q.device, workspace)
     _check(_lib.load().ccinfer_decode_attention_write_kv(
         _ptr(q), _ptr(k_new), _ptr(v_new), _ptr(k_cache), _ptr(v_cache), _ptr(block_table),
@@ -385,7 +394,7 @@ def decode_attention_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.
     _dev_tensor(output, torch.bfloat16, op)
     _require(output.shape == q.shape, op)
     mbpr = block_table.shape[1]
-    need = decode_workspace_size(b, mbpr, hq, hkv, d, cache_block_size)
+    need = _size(decode_workspace_size, b, mbpr, hq, hkv, d, cache_block_size)
     ws, ws_bytes = _workspace(need, q.device, workspace)
     _check(_lib.load().ccinfer_decode_attention_fp8(
         _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(k_scale), _ptr(v_scale), _ptr(block_table),
@@ -421,7 +430,7 @@ def prefill_attention_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch
     _dev_tensor(output, torch.bfloat16, op)
     _require(output.shape == q.shape, op)
     mbpr = block_table.shape[1]
-    need = prefill_workspace_size(b, total, mbpr, hq, hkv, d, cache_block_size)
+    need = _size(prefill_workspace_size, b, total, mbpr, hq, hkv, d, cache_block_size)
     ws, ws_bytes = _workspace(need, q.device, workspace)
     args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(k_scale), _ptr(v_scale),
             _ptr(block_table), _ptr(query_start_loc), _ptr(context_lens), _ptr(output), b, total,
@@ -460,7 +469,7 @@ def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     _dev_tensor(output, torch.bfloat16, op)
     _require(output.shape == q.shape, op)
     mbpr = block_table.shape[1]
-    need = prefill_workspace_size(b, total, mbpr, hq, hkv, d, cache_block_size)
+    need = _size(prefill_workspace_size, b, total, mbpr, hq, hkv, d, cache_block_size)
     ws, ws_bytes = _workspace(need, q.device, workspace)
     args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), _ptr(query_start_loc),
             _ptr(context_lens), _ptr(output), b, total, mbpr, hq, hkv, d, cache_block_size,
