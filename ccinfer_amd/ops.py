@@ -239,6 +239,15 @@ def _workspace(nbytes: int, device, workspace: Optional[torch.Tensor]):
     return torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes
 
 
+def _prefill_workspace(nbytes: int, device, workspace: Optional[torch.Tensor]):
+    """_workspace for the prefill calls, which also run in a workspace without the memory for
+    split tiles that the size query counts in: the call itself refuses one that is too small."""
+    if nbytes == 0 or workspace is None:
+        return _workspace(nbytes, device, workspace)
+    _require(workspace.is_cuda, "workspace")
+    return workspace, workspace.numel() * workspace.element_size()
+
+
 def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                      block_table: torch.Tensor, context_lens: torch.Tensor,
                      output: Optional[torch.Tensor] = None, cache_block_size: int = 16,
@@ -431,7 +440,7 @@ def prefill_attention_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch
     _require(output.shape == q.shape, op)
     mbpr = block_table.shape[1]
     need = _size(prefill_workspace_size, b, total, mbpr, hq, hkv, d, cache_block_size)
-    ws, ws_bytes = _workspace(need, q.device, workspace)
+    ws, ws_bytes = _prefill_workspace(need, q.device, workspace)
     args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(k_scale), _ptr(v_scale),
             _ptr(block_table), _ptr(query_start_loc), _ptr(context_lens), _ptr(output), b, total,
             mbpr, hq, hkv, d, cache_block_size, _ptr(ws), ws_bytes, _stream())
@@ -470,7 +479,7 @@ def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     _require(output.shape == q.shape, op)
     mbpr = block_table.shape[1]
     need = _size(prefill_workspace_size, b, total, mbpr, hq, hkv, d, cache_block_size)
-    ws, ws_bytes = _workspace(need, q.device, workspace)
+    ws, ws_bytes = _prefill_workspace(need, q.device, workspace)
     args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), _ptr(query_start_loc),
             _ptr(context_lens), _ptr(output), b, total, mbpr, hq, hkv, d, cache_block_size,
             _ptr(ws), ws_bytes, _stream())
