@@ -52,6 +52,7 @@
 #include "attn_common.hpp"
 #include "decode_core.hpp"
 #include "kernels.hpp"
+#include "prefill_split.hpp"
 
 namespace ccinfer::hipk {
 namespace {
@@ -1074,16 +1075,14 @@ __global__ __launch_bounds__(64 * GroupShape<D>::kWaves) void decode_group_kerne
         [&](int w) { return lds_o + w * kMaxG * D; }, lds_m, lds_l);
 }
 
-// One wavefront per (item, q_head) row with more than one split: log-sum-exp merge.
+// One wavefront (wi) per (item, q_head) row with more than one split: log-sum-exp merge.
 template <int D>
-__global__ __launch_bounds__(256) void decode_merge_kernel(
+__device__ __forceinline__ void merge_item_row(
     __bf16* __restrict__ out, const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
-    const MergeDesc* __restrict__ desc, ItemArgs items, int hq, int dr,
+    const MergeDesc* __restrict__ desc, const ItemArgs& items, int hq, int dr,
     const int32_t* __restrict__ flat_idx, int slots, const float* __restrict__ sh_o,
-    const float* __restrict__ sh_ml, int sh_k) {
+    const float* __restrict__ sh_ml, int sh_k, int wi) {
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wi = blockIdx.x * kWavesPerGroup + wave;
     const int head = wi % hq;
     const int item = wi / hq;
     if (item >= items.num_items) return;
@@ -1107,6 +1106,34 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(
     if (d.ns <= 1) return;  // invalid row, or written directly by the split kernel
     merge_row<D>(ws_o, ws_ml, d.base, static_cast<int>(d.ns), items.eps,
                  out + (static_cast<int64_t>(qrow) * hq + head) * dr, lane, dr);
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void decode_merge_kernel(
+    __bf16* __restrict__ out, const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
+    const MergeDesc* __restrict__ desc, ItemArgs items, int hq, int dr,
+    const int32_t* __restrict__ flat_idx, int slots, const float* __restrict__ sh_o,
+    const float* __restrict__ sh_ml, int sh_k) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    merge_item_row<D>(out, ws_o, ws_ml, desc, items, hq, dr, flat_idx, slots, sh_o, sh_ml, sh_k,
+                      blockIdx.x * kWavesPerGroup + wave);
+}
+
+// The merge of a prefill's decode items (the first row_wgs workgroups) and of its split tiles:
+// the host cannot tell whether the tiles split or the batch has decode items, so each merge is
+// often empty, and an empty launch costs 1-2 us. TD, TPad: the tile kernel's.
+template <int D, int TD, bool TPad>
+__global__ __launch_bounds__(256) void decode_merge_tiles_kernel(
+    __bf16* __restrict__ out, const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
+    const MergeDesc* __restrict__ desc, ItemArgs items, int hq, int dr,
+    const int32_t* __restrict__ flat_idx, int slots, int row_wgs, ptile::TileMerge t) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wg = blockIdx.x;
+    if (wg < row_wgs)
+        merge_item_row<D>(out, ws_o, ws_ml, desc, items, hq, dr, flat_idx, slots, nullptr, nullptr,
+                          0, wg * kWavesPerGroup + wave);
+    else
+        ptile::merge_tile_pieces<TD, TPad>(t, (wg - row_wgs) * kWavesPerGroup + wave);
 }
 
 struct DecodeWs {
@@ -1172,7 +1199,9 @@ hipError_t launch_decode(const void* q, const void* k_cache, const void* v_cache
                          const int32_t* block_table, const int32_t* context_lens, void* output,
                          const ItemArgs& it, int mbpr, int hq, int hkv, const DecodePlan& plan,
                          void* workspace, hipStream_t stream, int dr,
-                         const SharedParts& shared = SharedParts{}) {
+                         const SharedParts& shared = SharedParts{},
+                         DecodePart part = DecodePart::kAll,
+                         const ptile::TileMerge* tail = nullptr) {
     const float scale_log2 = kLog2e / sqrtf(static_cast<float>(dr));
     // Query groups larger than one MFMA N-tile run as `rep` virtual kv heads of hq / hkv /
     // rep query heads each; virtual head v reads cache head v / rep.
@@ -1182,7 +1211,8 @@ hipError_t launch_decode(const void* q, const void* k_cache, const void* v_cache
     // (head dim 96: neighbouring kv heads' rows share lines) read lines more than once:
     // those loads stay in L2.
     const bool tl = kPad || rep > 1 || kU != 0 || D % 64 != 0;
-    if (plan.group) {
+    const bool merge = !plan.group && (plan.flat || plan.splits > 1 || shared.o != nullptr);
+    if (plan.group && part != DecodePart::kMerge) {
         const int64_t groups = static_cast<int64_t>(it.num_items) * hkv;
         auto go = [&](auto tl_tag) {
             decode_group_kernel<D, F8, kPad, decltype(tl_tag)::value, kU>
@@ -1197,13 +1227,27 @@ hipError_t launch_decode(const void* q, const void* k_cache, const void* v_cache
             go(std::false_type{});
         return hipGetLastError();
     }
+    DecodeWs w{};
+    if (merge) w = carve(workspace, partial_rows(it.num_items, hq, plan), D, it.num_items, hq);
+    const int64_t rows = static_cast<int64_t>(it.num_items) * hq;
+    const int mgrid = merge ? static_cast<int>((rows + kWavesPerGroup - 1) / kWavesPerGroup) : 0;
+    if (part == DecodePart::kMerge) {
+        if constexpr (kU == 0 && D <= 128) {
+            if (tail != nullptr) {
+                constexpr int TD = D <= 64 ? 64 : 128;
+                decode_merge_tiles_kernel<D, TD, kPad || D != TD>
+                    <<<mgrid + ptile::tile_merge_wgs(*tail, TD), 256, 0, stream>>>(
+                        static_cast<__bf16*>(output), w.o, w.ml, w.desc, it, hq, dr,
+                        plan.flat_index ? w.index : nullptr, plan.slots, mgrid, *tail);
+                return hipGetLastError();
+            }
+        }
+        return hipErrorInvalidValue;
+    }
     const int64_t waves = plan.flat
                               ? static_cast<int64_t>(plan.slots) * hkv
                               : static_cast<int64_t>(it.num_items) * hkv * plan.splits;
     const int grid = static_cast<int>((waves + kWavesPerGroup - 1) / kWavesPerGroup);
-    const bool merge = plan.flat || plan.splits > 1 || shared.o != nullptr;
-    DecodeWs w{};
-    if (merge) w = carve(workspace, partial_rows(it.num_items, hq, plan), D, it.num_items, hq);
     if (plan.flat_index) {
         decode_flat_index_kernel<<<1, 1024, 0, stream>>>(context_lens, it, mbpr, plan.wave_target,
                                                          plan.slots, plan.flat_snap ? 1 : 0,
@@ -1253,9 +1297,7 @@ hipError_t launch_decode(const void* q, const void* k_cache, const void* v_cache
         go(std::false_type{}, std::false_type{});
     }
     hipError_t err = hipGetLastError();
-    if (err != hipSuccess || !merge) return err;
-    const int64_t rows = static_cast<int64_t>(it.num_items) * hq;
-    const int mgrid = static_cast<int>((rows + kWavesPerGroup - 1) / kWavesPerGroup);
+    if (err != hipSuccess || !merge || part == DecodePart::kSplits) return err;
     decode_merge_kernel<D><<<mgrid, 256, 0, stream>>>(static_cast<__bf16*>(output), w.o, w.ml,
                                                       w.desc, it, hq, dr,
                                                       plan.flat_index ? w.index : nullptr,
@@ -1405,7 +1447,7 @@ hipError_t decode_attention(const void* q, const void* k_cache, const void* v_ca
     launch_decode<DD, false, PP, UU>(q, k_cache, v_cache, nullptr, nullptr, block_table,      \
                                      context_lens, output, it, max_blocks_per_req,            \
                                      num_q_heads, num_kv_heads, plan, workspace, stream,      \
-                                     head_dim)
+                                     head_dim, SharedParts{}, items.part, items.tail)
 #define CCI_DECODE(DD, PP)                                                                   \
     return unaligned == 0 ? CCI_DECODE_U(DD, PP, 0)                                           \
                           : unaligned == 4 ? CCI_DECODE_U(DD, PP, 4) : CCI_DECODE_U(DD, PP, 2)
@@ -1446,15 +1488,18 @@ hipError_t decode_attention_fp8(const void* q, const void* k_cache, const void* 
         case 64:
             return launch_decode<64, true, false>(q, k_cache, v_cache, k_scale, v_scale, block_table,
                                            context_lens, output, it, max_blocks_per_req,
-                                           num_q_heads, num_kv_heads, plan, workspace, stream, 64);
+                                           num_q_heads, num_kv_heads, plan, workspace, stream, 64,
+                                           SharedParts{}, items.part, items.tail);
         case 128:
             return launch_decode<128, true, false>(q, k_cache, v_cache, k_scale, v_scale, block_table,
                                             context_lens, output, it, max_blocks_per_req,
-                                            num_q_heads, num_kv_heads, plan, workspace, stream, 128);
+                                            num_q_heads, num_kv_heads, plan, workspace, stream, 128,
+                                           SharedParts{}, items.part, items.tail);
         case 256:
             return launch_decode<256, true, false>(q, k_cache, v_cache, k_scale, v_scale, block_table,
                                             context_lens, output, it, max_blocks_per_req,
-                                            num_q_heads, num_kv_heads, plan, workspace, stream, 256);
+                                            num_q_heads, num_kv_heads, plan, workspace, stream, 256,
+                                           SharedParts{}, items.part, items.tail);
         default:
             return hipErrorInvalidValue;
     }

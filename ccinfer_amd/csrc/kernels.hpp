@@ -61,6 +61,13 @@ int decode_mfma_dim(int head_dim);
 // The same for an fp8 cache: head dims 64, 128 and 256 only.
 bool decode_fp8_supported(int num_q_heads, int num_kv_heads, int head_dim, int block_size);
 
+namespace ptile {
+struct TileMerge;
+}
+
+// Which launches of a decode run: all, those before its merge, or the merge.
+enum class DecodePart { kAll, kSplits, kMerge };
+
 // Query rows to attend, described either densely (item i is request i, query row i)
 // or through a device list written by the prefill planner.
 struct DecodeItems {
@@ -76,6 +83,10 @@ struct DecodeItems {
     const void* new_k = nullptr;
     const void* new_v = nullptr;
     int max_slots = 0;
+    DecodePart part = DecodePart::kAll;
+    // With part = kMerge: a tile merge of the prefill that the merge launch takes along (it is
+    // launched for that also where the plan has no merge); head dims up to 128.
+    const ptile::TileMerge* tail = nullptr;
 };
 
 // Request b's new token (bf16 [B][Hkv][head_dim]) into the cache slot of its last position

@@ -11,7 +11,8 @@
 // Launch plan (all on the caller's stream, no host sync, no allocation):
 //   1. plan kernel (one workgroup): reads query_start_loc / context_lens, emits the list of
 //      query tiles sorted longest-first (counting sort on the number of visible keys), and
-//      the list of single-token requests (decode items of a mixed batch).
+//      the list of single-token requests (decode items of a mixed batch). Not launched where
+//      neither list is read (see 2 and 3).
 //   2. tile kernel: one workgroup (8 wavefronts) per (query tile, kv_head, head group).
 //      Each wavefront owns 32 query rows of one q-head (16 for head_dim 256); the
 //      workgroup covers Hq/Hkv heads that share one KV head so every K/V tile staged in LDS
@@ -22,8 +23,8 @@
 //      and every O accumulator of a lane belongs to one query row (lane-local rescale).
 //      Tiles entirely above the causal diagonal are skipped; masking only runs on the
 //      diagonal / ragged tiles. Launches that fill at most half the CUs split the tiles' key
-//      ranges over more workgroups, whose partial rows a merge kernel combines (see "Split
-//      tiles").
+//      ranges over more workgroups, which find their pieces themselves, and a merge combines
+//      their partial rows (prefill_split.hpp).
 //   3. single-token requests run with prefill semantics (no 1e-6 in the denominator, bad
 //      rows left untouched). Batches (bf16 or fp8) of at most 1024 (request, virtual kv head) groups with
 //      table rows of at most 2048 positions run them in extra workgroups at the front of the
@@ -37,11 +38,13 @@
 #include "attn_common.hpp"
 #include "decode_core.hpp"
 #include "kernels.hpp"
+#include "prefill_split.hpp"
 
 namespace ccinfer::hipk {
 namespace {
 
-constexpr int kKeysPerTile = 64;
+using namespace ptile;
+
 constexpr int kThreads = 512;     // tile kernel: 8 wavefronts, 2 per SIMD
 constexpr int kWaves = kThreads / 64;
 constexpr int kBlock = 16;        // cache block size of the fast path
@@ -59,35 +62,11 @@ struct PrefillShape {
     static constexpr int kLoadsPerThread = kKeysPerTile * kCPR / kThreads;  // per K or V
 };
 
-// Heads per workgroup: the 8 wavefronts split as HPW heads x (8/HPW) row groups.
-__host__ __device__ inline int heads_per_wg(int G) {
-    return (G % 4 == 0) ? 4 : ((G % 2 == 0) ? 2 : 1);
-}
-
 // One workgroup's work (times the head units): query rows from t0 of request req against its
 // whole visible range.
 struct TileEntry {
     int req;
     int t0;
-};
-
-// The same where tiles may be split (see SplitPlan): against the 64-key tiles [kt0, kt1) of the
-// range. slot < 0: all of it, written to the output; else one piece, written to partial slot
-// `slot`.
-struct SplitEntry {
-    int req;
-    int t0;
-    int kt0;
-    int kt1;
-    int slot;
-};
-
-// A query tile cut into `pieces` pieces, whose partials are in slots slot0 .. + pieces.
-struct SplitTile {
-    int req;
-    int t0;
-    int slot0;
-    int pieces;
 };
 
 // Inclusive prefix sum over the 64 lanes of a wavefront (shuffles, no LDS).
@@ -133,69 +112,23 @@ __device__ void block_inclusive_scan(int* a, int n, int* part) {
 }
 
 // ---------------------------------------------------------------------------
-// Split tiles. A tile workgroup walks its whole visible range, so a launch with fewer
-// workgroups than CUs leaves CUs idle for as long as its longest tile takes. Where the batch
-// fills at most half of them, the planner cuts the longest tile into c = 256 / workgroups
-// pieces (c workgroups for every one of that size are one round of the chip), the others into
-// pieces of at most that length P, never under kSplitMinTiles. Each piece is a workgroup of its
-// own that leaves unnormalised fp32 rows and (m, l) pairs for prefill_merge_kernel.
-// A key tile takes ~1.8 us at head dim 128 (half that at 64), while a split costs the merge
-// (5-10 us) and a prologue per piece: tiles are split where that saves at least kSplitGain of
-// them. Measured, unsplit -> split: 1 x (12,345 cached + 1,024 new) 32q/8kv 280 -> 210 us, 2 x
-// (20,000 + 16) 395 -> 66, 1 x (2,000 + 512) 16q/8kv 69 -> 46, 1 x 2,048 16q/8kv 57 -> 48, 1 x
-// (900 + 200) 37.5 -> 33, fp8 1 x (8,000 + 1,024) 252 -> 166; with 176-280 workgroups (2 x
-// (1,000 + 700), 1 x 1,536 and 1 x 2,048 at 32q/8kv) pieces of unequal rounds and the merge lost
-// 6-8 us, hence the half; at savings of 8-12 key tiles the two sides are even. An estimate of
-// each of 16 piece lengths from a histogram of the pieces, on the device, found little better
-// lengths and took 5 us itself.
-// ---------------------------------------------------------------------------
-constexpr int kSplitCus = 256;
-constexpr int kSplitMinTiles = 4;
-constexpr int kSplitGain = 14;  // key tiles at head dim 128
-
-struct SplitPlan {
-    SplitTile* split;     // the split tiles (counts[2] of them)
-    SplitEntry* entries;  // the work list, in place of TileEntry's
-    int units;         // workgroups per tile; 0: tiles are not split
-    int gain;          // key tiles a split has to save
-    int key_cap;       // positions a table row can hold
-};
-
-// The piece length P for `tiles` query tiles whose longest has `longest` key tiles (a huge one:
-// no split). The host calls it with the fewest tiles and the longest table row possible, to
-// see whether a launch may split at all. At most kSplitCus / units pieces come out: every tile
-// has at most c of them.
-__host__ __device__ inline int split_length(int tiles, int units, int longest, int gain) {
-    const int wgs = tiles * units;
-    const int c = wgs > 0 ? kSplitCus / wgs : kSplitCus;
-    if (c < 2) return 0x7fffffff;
-    int P = (longest + c - 1) / c;
-    if (P < kSplitMinTiles) P = kSplitMinTiles;
-    return longest - P >= gain ? P : 0x7fffffff;
-}
-
-// ---------------------------------------------------------------------------
 // Planner: one workgroup of 1024 threads.
-// ws layout: counts[0] = #tile entries, counts[1] = #decode items, counts[2] = #split tiles;
-// tiles[max_tiles] (kSplit: sp.entries instead); dec[B].
+// ws layout: counts[0] = #tiles, counts[1] = #decode items; tiles[max_tiles]; dec[B].
 // split_dec: single-token requests become decode items (else one-row tiles).
 // kBig: more than kMaxPlanRequests requests; the per-request arrays then live in the
 // workspace (big_ntiles / big_scan, B ints each) instead of LDS.
 // ---------------------------------------------------------------------------
-// kSplit: tiles may be split (never with kBig); a kernel of its own, since the planner's time
-// grows with its code (one cold workgroup: +0.7 us for the split's).
-template <bool kBig, bool kSplit>
+template <bool kBig>
 __global__ __launch_bounds__(1024) void prefill_plan_kernel(
     const int32_t* __restrict__ qsl, const int32_t* __restrict__ context_lens, int batch_size,
     int total_tokens, int tile_tokens, int32_t* __restrict__ counts,
     TileEntry* __restrict__ tiles, int32_t* __restrict__ dec_req, uint32_t* __restrict__ zero_row,
-    int zero_words, int* __restrict__ big_ntiles, int* __restrict__ big_scan, int split_dec,
-    SplitPlan sp) {
+    int zero_words, int* __restrict__ big_ntiles, int* __restrict__ big_scan, int split_dec) {
     __shared__ int lds_ntiles[kBig ? 1 : kMaxPlanRequests];
     __shared__ int lds_scan[kBig ? 1 : kMaxPlanRequests];
-    // Each request's query rows and cached prefix, read once (the bucket pass and the
+    // Each request's query length and cached prefix, read once (the bucket pass and the
     // scatter pass need them again).
-    __shared__ int lds_rows[kBig ? 1 : kMaxPlanRequests];
+    __shared__ int lds_qlen[kBig ? 1 : kMaxPlanRequests];
     __shared__ int lds_prefix[kBig ? 1 : kMaxPlanRequests];
     int* s_ntiles = kBig ? big_ntiles : lds_ntiles;
     int* s_scan = kBig ? big_scan : lds_scan;
@@ -204,11 +137,7 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(
     __shared__ int s_part[16];
     __shared__ int s_ndec;
     __shared__ int s_total;
-    __shared__ SplitTile s_split[kSplit ? kSplitCus / 2 : 1];  // two pieces or more each
-    __shared__ int s_cost[kSplit ? kSplitCus / 2 : 1];
-    __shared__ int s_costmax, s_entries, s_slots, s_nsplit;
     const int tid = threadIdx.x;
-    if (kSplit && tid == 0) s_costmax = s_entries = s_slots = s_nsplit = 0;
     for (int i = tid; i < zero_words; i += blockDim.x) zero_row[i] = 0u;  // staging's zero row
     for (int i = tid; i < kBuckets; i += blockDim.x) s_hist[i] = 0;
     if (tid == 0) s_ndec = 0;
@@ -228,7 +157,7 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(
         const int rows = qe - (qb > 0 ? qb : 0);
         const int prefix = context_lens[b] - qlen;
         if constexpr (!kBig) {
-            lds_rows[b] = rows;
+            lds_qlen[b] = qlen;
             lds_prefix[b] = prefix;
         }
         int n = 0;
@@ -271,51 +200,18 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(
         *b_out = lo;
         *r_out = t - (s_scan[lo] - s_ntiles[lo]);
     };
-    // 64-key tiles of query tile r of request b, as the tile kernel counts them
-    auto cost_of = [&](int b, int r) {
-        int rows, prefix;
-        if constexpr (kBig) {
-            const int qb = qsl[b], qe = qsl[b + 1];
-            rows = (qe < total_tokens ? qe : total_tokens) - qb;
-            prefix = context_lens[b] - (qe - qb);
-        } else {
-            rows = lds_rows[b];
-            prefix = lds_prefix[b];
-        }
+    auto bucket_of = [&](int b, int r) {
+        const int qlen = kBig ? qsl[b + 1] - qsl[b] : lds_qlen[b];
+        const int prefix = kBig ? context_lens[b] - qlen : lds_prefix[b];
         int last = (r + 1) * tile_tokens;
-        if (last > rows) last = rows;
-        const int keys = min(prefix + last, sp.key_cap);
-        return (keys + kKeysPerTile - 1) / kKeysPerTile;
-    };
-    auto bucket_of = [&](int cost) {
+        if (last > qlen) last = qlen;
+        const int cost = (prefix + last) >> 6;
         return kBuckets - 1 - (cost < kBuckets - 1 ? cost : kBuckets - 1);
     };
-    int P = 0x7fffffff;  // key tiles a piece may have
-    if constexpr (kSplit) {
-        int c = 0;
-        for (int t = tid; t < total; t += blockDim.x) {
-            int b, r;
-            locate(t, &b, &r);
-            c = max(c, cost_of(b, r));
-        }
-        if (c > 0) atomicMax(&s_costmax, c);
-        __syncthreads();
-        P = split_length(total, sp.units, s_costmax, sp.gain);
-    }
-    // A split tile's first cost % c pieces have cost / c + 1 key tiles, the others cost / c.
     for (int t = tid; t < total; t += blockDim.x) {
         int b, r;
         locate(t, &b, &r);
-        const int cost = cost_of(b, r);
-        if (!kSplit || cost <= P) {
-            atomicAdd(&s_hist[bucket_of(cost)], 1);
-        } else {
-            const int c = (cost + P - 1) / P;
-            const int len = cost / c, more = cost - len * c;
-            if (more > 0) atomicAdd(&s_hist[bucket_of(len + 1)], more);
-            atomicAdd(&s_hist[bucket_of(len)], c - more);
-            atomicAdd(&s_entries, c - 1);
-        }
+        atomicAdd(&s_hist[bucket_of(b, r)], 1);
     }
     __syncthreads();
     // Exclusive scan of the histogram -> first slot of each bucket.
@@ -327,40 +223,12 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(
     for (int t = tid; t < total; t += blockDim.x) {
         int b, r;
         locate(t, &b, &r);
-        const int cost = cost_of(b, r);
-        if (!kSplit || cost <= P) {
-            const int pos = atomicAdd(&s_hist[bucket_of(cost)], 1);
-            if (kSplit)
-                sp.entries[pos] = SplitEntry{b, r * tile_tokens, 0, cost, -1};
-            else
-                tiles[pos] = TileEntry{b, r * tile_tokens};
-        } else {
-            const int c = (cost + P - 1) / P;
-            const int i = atomicAdd(&s_nsplit, 1);
-            const SplitTile st{b, r * tile_tokens, atomicAdd(&s_slots, c), c};
-            sp.split[i] = st;
-            s_split[i] = st;
-            s_cost[i] = cost;
-        }
-    }
-    if constexpr (kSplit) {
-        __syncthreads();
-        // one wavefront per split tile, one lane per piece
-        for (int i = tid >> 6; i < s_nsplit; i += blockDim.x >> 6) {
-            const SplitTile st = s_split[i];
-            const int len = s_cost[i] / st.pieces, more = s_cost[i] - len * st.pieces;
-            for (int k = tid & 63; k < st.pieces; k += 64) {
-                const int k0 = k * len + min(k, more);
-                const int size = len + (k < more ? 1 : 0);
-                const int pos = atomicAdd(&s_hist[bucket_of(size)], 1);
-                sp.entries[pos] = SplitEntry{st.req, st.t0, k0, k0 + size, st.slot0 + k};
-            }
-        }
+        const int pos = atomicAdd(&s_hist[bucket_of(b, r)], 1);
+        tiles[pos] = TileEntry{b, r * tile_tokens};
     }
     if (tid == 0) {
-        counts[0] = total + (kSplit ? s_entries : 0);
+        counts[0] = total;
         counts[1] = s_ndec;
-        if (kSplit) counts[2] = s_nsplit;
     }
 }
 
@@ -538,7 +406,6 @@ __device__ __forceinline__ bf16x8 load_vt(const __bf16* lv, int h2, int n, int l
 // stay <= 2^8 (pipelined kernel: below 2) and sums of them fit fp32 comfortably; acc and l always share one reference
 // max, so the final acc / l is exact whatever the reference.
 constexpr float kRescaleSlack = 8.0f;
-constexpr float kMaxInit = -1.0e30f;
 // Pipelined kernel: how far above a row's max the reference is set, so that probabilities
 // start at or below 2^-6 and the row may grow by 7 before one reaches 2.
 constexpr float kRefHead = 6.0f;
@@ -891,16 +758,6 @@ __global__ __launch_bounds__(kThreads) void prefill_tile_kernel(
 // 518 us (1.07 -> 1.13), 8 x (512 + 1,536) 144.5 -> 141 us, head dim 64 8 x (4,096 + 1,024)
 // 350 -> 335 us, fp8 8 x (2,048 + 1,024) 195 -> 189 us.
 // ---------------------------------------------------------------------------
-template <int D>
-struct PipeShape {
-    static constexpr int kRows = 32;                     // query rows per wavefront
-    static constexpr int kWaves = 8;
-    static constexpr int kThreads = 64 * kWaves;
-    static constexpr int kCPR = D / 8;                   // 16-byte chunks per K/V row
-    static constexpr int kLoads = kKeysPerTile * kCPR / kThreads;  // per K or V
-    static_assert(kKeysPerTile * kCPR % kThreads == 0, "staging must split evenly");
-};
-
 __host__ __device__ constexpr bool pipe_head_dim(int d) { return d == 64 || d == 128; }
 
 // F8: the cache holds OCP E4M3 bytes with row scales (k_scale / v_scale). A tile's bytes are
@@ -922,8 +779,8 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
                          const int32_t* __restrict__ counts, const TileEntry* __restrict__ tiles,
                          int total_tokens, int mbpr, int hq, int hkv, float scale_log2,
                          int dr, dcore::ItemArgs dec_items, int dec_wgs, int dec_hkv,
-                         int dec_rep, const SplitEntry* __restrict__ entries,
-                         float* __restrict__ part_o, float* __restrict__ part_ml) {
+                         int dec_rep, SplitRule split, float* __restrict__ part_o,
+                         float* __restrict__ part_ml) {
     static_assert(!(F8 && kPad), "fp8 runs the native head dims only");
     const int ds = kPad ? dr : D;  // row stride of q / cache / output (elements)
     using Sh = PipeShape<D>;
@@ -975,27 +832,28 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     const int WPH = kPipeWaves / HPW;
     const int U = hkv * (G / HPW);
     const int tile_idx = bid / U;
-    if (tile_idx >= counts[0]) return;
     const int u = bid % U;
     const int kvh = u / (G / HPW);
     const int hg = u % (G / HPW);
-    SplitEntry te{0, 0, 0, 0x7fffffff, -1};
-    if (entries != nullptr) {
-        te = entries[tile_idx];
+    // A launch that may split has the pieces of a tile side by side; else the planner's list.
+    TilePiece te;
+    if (split.batch > 0) {
+        const SplitPlan plan = split_plan(split);
+        const int tile = __builtin_amdgcn_readfirstlane(tile_idx / plan.per);
+        if (!split_piece(split, plan, tile, tile_idx - tile * plan.per, &te)) return;
     } else {
+        if (tile_idx >= counts[0]) return;
         const TileEntry whole = tiles[tile_idx];
-        te.req = whole.req;
-        te.t0 = whole.t0;
+        const int first = qsl[whole.req];
+        const int end = qsl[whole.req + 1];
+        te = TilePiece{whole.req, first, min(end, total_tokens) - first,
+                       context_lens[whole.req] - (end - first), whole.t0, 0, kWhole, 0, 1};
     }
     const int req = te.req;
     const int t0 = te.t0;
-
-    const int qb = qsl[req];
-    const int qlen = qsl[req + 1] - qb;
-    const int ctx = context_lens[req];
-    const int prefix = ctx - qlen;
-    const int qe = min(qb + qlen, total_tokens);
-    const int rows = qe - qb;
+    const int qb = te.qb;
+    const int rows = te.rows;
+    const int prefix = te.prefix;
     const int TT = WPH * kPipeRows;
     const int kv_end = prefix + min(t0 + TT, rows);  // keys past it are masked for every row
     // Positions past the table row are invalid: no tile needs to reach them.
@@ -1702,9 +1560,9 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     // Epilogue: lane (c, h) holds O[tw + c][32 n + 8 i + 4 h + r] = acc[n][4 i + r].
     {
         const float l_tot = (lane & 16) ? lsum[1] : lsum[0];
-        if (te.slot >= 0) {
+        if (te.pieces > 1) {
             // A piece of a split tile: the lanes' accumulators as they are, 16 bytes a lane
-            // and store (a row-major layout would scatter them), for prefill_merge_kernel.
+            // and store (a row-major layout would scatter them), for the merge.
             const int64_t wv = (static_cast<int64_t>(te.slot) * U + u) * kPipeWaves + wave;
             f32x4* po = reinterpret_cast<f32x4*>(part_o) + wv * (NT2 * 4 * 64) + lane;
 #pragma unroll
@@ -1736,72 +1594,10 @@ void prefill_pipe_kernel(const __bf16* __restrict__ q, const void* __restrict__ 
     }
 }
 
-// Log-sum-exp merge of the pieces of split tiles (counts[2] of them). One wavefront per
-// (split tile, unit, wavefront of the tile kernel, 32-dim block n): it reads the partials in
-// the tile kernel's own lane layout, so every load is a whole kilobyte, and stores the rows as
-// that kernel's epilogue does.
 template <int D, bool kPad>
-__global__ __launch_bounds__(256) void prefill_merge_kernel(
-    __bf16* __restrict__ out, const float* __restrict__ part_o,
-    const float* __restrict__ part_ml, const int32_t* __restrict__ counts,
-    const SplitTile* __restrict__ split, const int32_t* __restrict__ qsl, int total_tokens,
-    int hq, int hkv, int dr) {
-    constexpr int kPipeWaves = PipeShape<D>::kWaves;
-    constexpr int kPipeRows = PipeShape<D>::kRows;
-    constexpr int NT2 = D / 32;
-    const int ds = kPad ? dr : D;
-    const int G = hq / hkv;
-    const int HPW = heads_per_wg(G);
-    const int WPH = kPipeWaves / HPW;
-    const int U = hkv * (G / HPW);
-    const int lane = threadIdx.x & 63;
-    const int wi = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n = wi % NT2;
-    const int wave = wi / NT2 % kPipeWaves;
-    const int u = wi / (NT2 * kPipeWaves) % U;
-    const int si = wi / (NT2 * kPipeWaves * U);
-    if (si >= counts[2]) return;
-    const SplitTile st = split[si];
-    const int qb = qsl[st.req];
-    const int rows = min(qsl[st.req + 1], total_tokens) - qb;
-    const int tw = st.t0 + (wave % WPH) * kPipeRows;
-    if (tw >= rows) return;
-    const int q_head = u / (G / HPW) * G + u % (G / HPW) * HPW + wave / WPH;
-    const int c32 = lane & 31;
-    const int h32 = lane >> 5;
-    const int64_t wv0 = (static_cast<int64_t>(st.slot0) * U + u) * kPipeWaves + wave;
-    const int64_t step = static_cast<int64_t>(U) * kPipeWaves;
-    float mmax = kMaxInit;
-#pragma unroll 8
-    for (int p = 0; p < st.pieces; ++p)
-        mmax = fmaxf(mmax, part_ml[((wv0 + p * step) * kPipeRows + c32) * 2]);
-    f32x4 acc[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float l = 0.f;
-#pragma unroll 4
-    for (int p = 0; p < st.pieces; ++p) {
-        const int64_t wv = wv0 + p * step;
-        const f32x2 ml = *reinterpret_cast<const f32x2*>(part_ml + (wv * kPipeRows + c32) * 2);
-        const f32x4* po = reinterpret_cast<const f32x4*>(part_o) + wv * (NT2 * 4 * 64) +
-                          n * 4 * 64 + lane;
-        const float w = __builtin_amdgcn_exp2f(ml[0] - mmax);
-        l += ml[1] * w;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] = acc[i] + po[i * 64] * w;
-    }
-    const int tq = tw + c32;
-    if (tq >= rows) return;
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    __bf16* o = out + (static_cast<int64_t>(qb + tq) * hq + q_head) * ds;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        if (kPad && 32 * n + 8 * i + 4 * h32 >= dr) continue;  // padded dims
-        u32x2 w;
-        w[0] = pack_bf16x2(acc[i][0] * inv, acc[i][1] * inv);
-        w[1] = pack_bf16x2(acc[i][2] * inv, acc[i][3] * inv);
-        *reinterpret_cast<u32x2*>(o + 32 * n + 8 * i + 4 * h32) = w;
-    }
+__global__ __launch_bounds__(256) void prefill_merge_kernel(TileMerge t) {
+    merge_tile_pieces<D, kPad>(
+        t, blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
 }
 
 struct PrefillLayout {
@@ -1810,7 +1606,7 @@ struct PrefillLayout {
     int tile_tokens;
     int units;   // workgroups per query tile
     int gain;    // key tiles a split has to save
-    bool split;  // whether the planner may split tiles (given the memory for it)
+    bool split;  // whether the launch may split tiles (given the memory for it)
     DecodePlan plan;
 };
 
@@ -1839,20 +1635,19 @@ PrefillLayout prefill_layout(int batch_size, int total_query_tokens, int max_blo
     L.tile_tokens = tile_tokens_for(D, G);
     L.max_tiles = total_query_tokens / L.tile_tokens + batch_size;
     L.units = num_kv_heads * (G / heads_per_wg(G));
-    // Whether the planner may split tiles: the same rule for the fewest tiles these tokens can
+    // Whether the launch may split tiles: the same rule for the fewest tiles these tokens can
     // make (at least one a request: single-token requests make none, but a batch that has
     // many of those is not short of workgroups) and a table row full of positions. A split is
-    // then possible, not certain.
+    // then possible, not certain. max_tiles is then at most kSplitCus / units.
     L.gain = split_gain(D);
-    if (pipe_head_dim(D) && batch_size <= kMaxPlanRequests &&
-        split_length(std::max(batch_size, total_query_tokens / L.tile_tokens), L.units,
-                     row_key_tiles(max_blocks_per_req, block_size), L.gain) < 0x7fffffff)
-        L.split = true;
+    L.split = pipe_head_dim(D) && batch_size <= kSplitRequests &&
+              split_length(std::max(batch_size, total_query_tokens / L.tile_tokens), L.units,
+                           row_key_tiles(max_blocks_per_req, block_size), L.gain) != kWhole;
     L.plan = plan_decode_items(batch_size, num_q_heads, num_kv_heads, head_dim,
                                max_blocks_per_req * block_size, fp8);
     size_t off = 0;
     L.counts_off = off;
-    off = align256(off + 3 * sizeof(int32_t));
+    off = align256(off + 2 * sizeof(int32_t));
     L.zero_off = off;  // one all-zero K/V row (D bf16), rewritten by the planner
     off = align256(off + static_cast<size_t>(D) * 2);
     L.tiles_off = off;
@@ -1868,11 +1663,7 @@ PrefillLayout prefill_layout(int batch_size, int total_query_tokens, int max_blo
     return L;
 }
 
-// The memory of split tiles: their list, the work list (a batch that may split has at most
-// kSplitCus / 2 requests and as many whole tiles of its tokens, and kSplitCus pieces), then
-// the partial rows and (m, l) pairs of at most kSplitCus workgroups.
-constexpr size_t kSplitListBytes =
-    (kSplitCus / 2 * sizeof(SplitTile) + 2 * kSplitCus * sizeof(SplitEntry) + 255) & ~size_t{255};
+// The partial rows and (m, l) pairs of at most kSplitCus workgroups.
 constexpr size_t kSplitRows =
     static_cast<size_t>(kSplitCus) * PipeShape<64>::kWaves * PipeShape<64>::kRows;
 
@@ -1885,7 +1676,7 @@ hipError_t launch_tiles(const void* q, const void* k_cache, const void* v_cache,
                         int mbpr, int hq, int hkv, int block_size, const int32_t* counts,
                         const TileEntry* tiles, const void* zero_row, int max_tiles,
                         hipStream_t stream, int dr, int batch_size, bool fused_dec,
-                        const SplitPlan& sp, float* part_o, float* part_ml) {
+                        const SplitRule& split, float* part_o, float* part_ml) {
     const int G = hq / hkv;
     const int U = hkv * (G / heads_per_wg(G));
     const float scale_log2 = kLog2e / sqrtf(static_cast<float>(dr));
@@ -1902,23 +1693,14 @@ hipError_t launch_tiles(const void* q, const void* k_cache, const void* v_cache,
             it.singles_total = total_query_tokens;
             dec_wgs = batch_size * hkv * rep;
         }
-        const int max_entries = max_tiles + (sp.units > 0 ? kSplitCus / sp.units : 0);
-        const int64_t grid = static_cast<int64_t>(max_entries) * U + dec_wgs;
+        const int entries = split.batch > 0 ? kSplitCus / U : max_tiles;
+        const int64_t grid = static_cast<int64_t>(entries) * U + dec_wgs;
         prefill_pipe_kernel<D, F8, kPad>
             <<<static_cast<unsigned>(grid), PipeShape<D>::kThreads, 0, stream>>>(
             static_cast<const __bf16*>(q), k_cache, v_cache, k_scale, v_scale, block_table, qsl,
             context_lens,
             static_cast<__bf16*>(output), counts, tiles, total_query_tokens, mbpr, hq, hkv,
-            scale_log2, dr, it, dec_wgs, hkv * rep, rep,
-            sp.units > 0 ? sp.entries : nullptr, part_o, part_ml);
-        const hipError_t err = hipGetLastError();
-        if (err != hipSuccess || sp.units == 0) return err;
-        // four wavefronts a workgroup; a tile has 8 D / 32 U of them (a multiple of four)
-        const int64_t mwgs = static_cast<int64_t>(std::min(max_tiles, kSplitCus / 2 / U)) * U *
-                             (PipeShape<D>::kWaves * (D / 32) / 4);
-        prefill_merge_kernel<D, kPad><<<static_cast<unsigned>(mwgs), 256, 0, stream>>>(
-            static_cast<__bf16*>(output), part_o, part_ml, counts, sp.split, qsl,
-            total_query_tokens, hq, hkv, dr);
+            scale_log2, dr, it, dec_wgs, hkv * rep, rep, split, part_o, part_ml);
         return hipGetLastError();
     } else if constexpr (F8) {
         return hipErrorInvalidValue;  // fp8 has the pipelined path only
@@ -1955,7 +1737,7 @@ size_t prefill_split_bytes(int head_dim, int max_blocks_per_req, int block_size)
     if (!pipe_head_dim(D) ||
         row_key_tiles(max_blocks_per_req, block_size) < kSplitMinTiles + split_gain(D))
         return 0;
-    return 256 + kSplitListBytes + kSplitRows * (D + 2) * sizeof(float);
+    return 256 + kSplitRows * (D + 2) * sizeof(float);
 }
 
 size_t prefill_workspace_bytes(int batch_size, int total_query_tokens, int max_blocks_per_req,
@@ -2028,24 +1810,30 @@ hipError_t prefill_impl(const void* q, const void* k_cache, const void* v_cache,
     // memory for it.
     const size_t split_need = prefill_split_bytes(head_dim, max_blocks_per_req, block_size);
     const bool can_split = L.split && !fork && split_need > 0 && split_bytes >= split_need;
-    char* sws = reinterpret_cast<char*>(align256(reinterpret_cast<uintptr_t>(split_ws)));
-    SplitTile* split = reinterpret_cast<SplitTile*>(sws);
-    SplitEntry* entries = reinterpret_cast<SplitEntry*>(split + kSplitCus / 2);
-    float* part_o = reinterpret_cast<float*>(sws + kSplitListBytes);
+    float* part_o =
+        reinterpret_cast<float*>(align256(reinterpret_cast<uintptr_t>(split_ws)));
     float* part_ml = part_o + kSplitRows * Dk;
-    SplitPlan sp{split, entries, can_split ? L.units : 0, L.gain,
-                 static_cast<int>(std::min<int64_t>(
-                     static_cast<int64_t>(max_blocks_per_req) * block_size, 0x7fffffff))};
+    SplitRule split;
+    TileMerge merge;
+    if (can_split) {
+        split = SplitRule{query_start_loc, context_lens, batch_size, total_query_tokens,
+                          L.tile_tokens, L.units, L.gain,
+                          static_cast<int>(std::min<int64_t>(
+                              static_cast<int64_t>(max_blocks_per_req) * block_size, 0x7fffffff))};
+        merge = TileMerge{split, static_cast<__bf16*>(output), part_o, part_ml, num_q_heads,
+                          num_kv_heads, head_dim, L.max_tiles};
+    }
+    // Without the planner where nothing reads its lists: a launch that may split finds its tiles
+    // itself, and one with fused_dec its single-token requests.
     if (batch_size > kMaxPlanRequests) {
         int* big = reinterpret_cast<int*>(ws + L.big_off);
-        prefill_plan_kernel<true, false><<<1, 1024, 0, stream>>>(
+        prefill_plan_kernel<true><<<1, 1024, 0, stream>>>(
             query_start_loc, context_lens, batch_size, total_query_tokens, L.tile_tokens, counts,
-            tiles, dec, zero_row, decode_mfma_dim(head_dim) / 2, big, big + batch_size, 1, sp);
-    } else {
-        auto plan = sp.units > 0 ? prefill_plan_kernel<false, true> : prefill_plan_kernel<false, false>;
-        plan<<<1, 1024, 0, stream>>>(
+            tiles, dec, zero_row, decode_mfma_dim(head_dim) / 2, big, big + batch_size, 1);
+    } else if (!(can_split && fused_dec)) {
+        prefill_plan_kernel<false><<<1, 1024, 0, stream>>>(
             query_start_loc, context_lens, batch_size, total_query_tokens, L.tile_tokens, counts,
-            tiles, dec, zero_row, decode_mfma_dim(head_dim) / 2, nullptr, nullptr, 1, sp);
+            tiles, dec, zero_row, decode_mfma_dim(head_dim) / 2, nullptr, nullptr, 1);
     }
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
@@ -2063,7 +1851,9 @@ hipError_t prefill_impl(const void* q, const void* k_cache, const void* v_cache,
     items.query_start_loc = query_start_loc;
     items.denom_eps = 0.0f;
     items.zero_invalid = false;
-    auto launch_decode_items = [&](hipStream_t s) {
+    auto launch_decode_items = [&](hipStream_t s, DecodePart part, const TileMerge* tail) {
+        items.part = part;
+        items.tail = tail;
         if constexpr (F8)
             return decode_attention_fp8(q, k_cache, v_cache, k_scale, v_scale, block_table,
                                         context_lens, output, items, max_blocks_per_req,
@@ -2086,10 +1876,12 @@ hipError_t prefill_impl(const void* q, const void* k_cache, const void* v_cache,
         if (err != hipSuccess) return err;
         err = hipStreamWaitEvent(overlap->side, overlap->fork, 0);
         if (err != hipSuccess) return err;
-        err = launch_decode_items(overlap->side);
+        err = launch_decode_items(overlap->side, DecodePart::kAll, nullptr);
         if (err != hipSuccess) return join(err);
     } else if (!fused_dec) {
-        err = launch_decode_items(stream);
+        // The merge of a launch that may split goes with the decode items' merge, after the tiles.
+        err = launch_decode_items(stream, can_split ? DecodePart::kSplits : DecodePart::kAll,
+                                  nullptr);
         if (err != hipSuccess) return err;
     }
     const int D = decode_mfma_dim(head_dim);
@@ -2099,7 +1891,7 @@ hipError_t prefill_impl(const void* q, const void* k_cache, const void* v_cache,
                              query_start_loc, context_lens, output, total_query_tokens,      \
                              max_blocks_per_req, num_q_heads, num_kv_heads, block_size,      \
                              counts, tiles, zero_row, L.max_tiles, stream, head_dim,         \
-                             batch_size, fused_dec, sp, part_o, part_ml)
+                             batch_size, fused_dec, split, part_o, part_ml)
     if (F8 && pad) {
         err = hipErrorInvalidValue;  // fp8 runs the native head dims only
     } else {
@@ -2118,7 +1910,17 @@ hipError_t prefill_impl(const void* q, const void* k_cache, const void* v_cache,
         }
     }
 #undef CCI_TILES
-    return fork ? join(err) : err;
+    if (fork) return join(err);
+    if (err != hipSuccess || !can_split) return err;
+    if (!fused_dec) return launch_decode_items(stream, DecodePart::kMerge, &merge);
+    const int wgs = tile_merge_wgs(merge, D);
+    if (D == 128)
+        (pad ? prefill_merge_kernel<128, true> : prefill_merge_kernel<128, false>)
+            <<<wgs, 256, 0, stream>>>(merge);
+    else
+        (pad ? prefill_merge_kernel<64, true> : prefill_merge_kernel<64, false>)
+            <<<wgs, 256, 0, stream>>>(merge);
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -2157,7 +1959,7 @@ AnyLayout any_layout(int batch_size, int total_query_tokens, int num_q_heads, in
     L.max_tiles = total_query_tokens / L.tile_tokens + batch_size;
     size_t off = 0;
     L.counts_off = off;
-    off = align256(off + 3 * sizeof(int32_t));
+    off = align256(off + 2 * sizeof(int32_t));
     L.tiles_off = off;
     off = align256(off + static_cast<size_t>(L.max_tiles) * sizeof(TileEntry));
     L.dec_off = off;
@@ -2195,17 +1997,16 @@ hipError_t prefill_attention_any(const void* q, const void* k_cache, const void*
     int32_t* counts = reinterpret_cast<int32_t*>(ws + L.counts_off);
     TileEntry* tiles = reinterpret_cast<TileEntry*>(ws + L.tiles_off);
     int32_t* dec = reinterpret_cast<int32_t*>(ws + L.dec_off);
-    const SplitPlan whole{nullptr, nullptr, 0, 0, 0x7fffffff};
     // single-token requests run as one-row tiles (the decode kernels take 16-token blocks)
     if (batch_size > kMaxPlanRequests) {
         int* big = reinterpret_cast<int*>(ws + L.big_off);
-        prefill_plan_kernel<true, false><<<1, 1024, 0, stream>>>(
+        prefill_plan_kernel<true><<<1, 1024, 0, stream>>>(
             query_start_loc, context_lens, batch_size, total_query_tokens, L.tile_tokens, counts,
-            tiles, dec, nullptr, 0, big, big + batch_size, 0, whole);
+            tiles, dec, nullptr, 0, big, big + batch_size, 0);
     } else {
-        prefill_plan_kernel<false, false><<<1, 1024, 0, stream>>>(
+        prefill_plan_kernel<false><<<1, 1024, 0, stream>>>(
             query_start_loc, context_lens, batch_size, total_query_tokens, L.tile_tokens, counts,
-            tiles, dec, nullptr, 0, nullptr, nullptr, 0, whole);
+            tiles, dec, nullptr, 0, nullptr, nullptr, 0);
     }
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
