@@ -222,7 +222,8 @@ __device__ __forceinline__ void merge_tile_pieces(const TileMerge& t, int wi) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     float l = 0.f;
-    // kBatch pieces' loads in flight at a time (past the last piece: a repeat of it, weight 0)
+    // kBatch pieces' loads in flight at a time (past the last piece: a repeat of it, which is not
+    // added: a row that V made infinite would become NaN by 0 * Inf)
     constexpr int kBatch = 4;
     for (int p0 = 0; p0 < st.pieces; p0 += kBatch) {
         f32x2 ml[kBatch];
@@ -239,7 +240,8 @@ __device__ __forceinline__ void merge_tile_pieces(const TileMerge& t, int wi) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int x = 0; x < kBatch; ++x) {
-            const float w = p0 + x < st.pieces ? __builtin_amdgcn_exp2f(ml[x][0] - mmax) : 0.f;
+            if (p0 + x >= st.pieces) break;
+            const float w = __builtin_amdgcn_exp2f(ml[x][0] - mmax);
             l += ml[x][1] * w;
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[i] = acc[i] + o[x][i] * w;

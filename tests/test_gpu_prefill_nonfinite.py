@@ -105,3 +105,21 @@ def test_query_rows_are_independent(gpu, prefix, news, hq, hkv, d, bad):
                     assert (got[row, head] != got[row, head]).all()
                 got[row, head] = want[row, head]
                 assert_attn_close(got, want, f"{kind}, bad row {r} of {n}")
+
+
+@pytest.mark.parametrize("prefix,news,hq,hkv,d", WHOLE[1:2] + SPLIT + [
+    (1136, (64, 256), 4, 4, 128),
+    (2992, (129,), 8, 2, 96),
+])
+def test_infinite_value_row(gpu, prefix, news, hq, hkv, d):
+    """A cached V row of +Inf under finite scores makes every output +Inf (its probability is
+    positive, the other values finite), never NaN: no partial sum is multiplied by 0."""
+    w = _inputs(gpu, prefix, news, hq, hkv, d)
+    m = w.device_meta(gpu)
+    meta = (m["block_table"], m["query_start_loc"], m["context_lens"])
+    for pos in (0, prefix - 1):
+        say(f"infinite value row prefix={prefix} new={news} {hq}/{hkv} d={d} pos={pos}")
+        v = w.v_cache.clone()
+        for b in range(len(news)):
+            v[int(w.block_table[b, pos // 16]) * 16 + pos % 16] = INF
+        assert (f32(prefill_attention(w.q, w.k_cache, v, *meta)) == INF).all()
