@@ -65,9 +65,18 @@ def _dev_tensor(t: Optional[torch.Tensor], dtype: torch.dtype, op: str) -> None:
         raise CcinferError(INVALID_ARGUMENT, op)
 
 
-def _stream() -> int:
-    """The raw handle of torch's current stream (torch.cuda.current_stream().cuda_stream)."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+def _stream_reader():
+    """A function that gives the raw handle of torch's current stream: by the calls under
+    torch.cuda.current_stream() where this torch has them (they are not public names), else
+    through its stream object."""
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    device = getattr(torch._C, "_cuda_getDevice", None)
+    if raw is None or device is None:
+        return lambda: torch.cuda.current_stream().cuda_stream
+    return lambda: raw(device())
+
+
+_stream = _stream_reader()
 
 
 class SideStream:
