@@ -519,7 +519,7 @@ __device__ void merge_row(const float* __restrict__ ws_o, const float* __restric
 
 // Log-sum-exp merge of a row whose partials sit in two lists: ns split partials at `base`
 // of the workspace and sn shared-prefix partials at `sbase` of the shared area (the rows of
-// decode_attention_shared). A plain loop: these rows are few per launch.
+// decode_attention_shared; every row of a launch whose requests share a prefix).
 template <int D>
 __device__ void merge_row_two(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
                               int64_t base, int ns, const float* __restrict__ sh_o,
@@ -600,7 +600,8 @@ constexpr int kSharedMinTokens = 64;      // shorter common prefixes are not wor
 constexpr int kSharedMaxItems = 2048;     // the planner's hash table holds 2x this many keys
 constexpr int kSharedHash = 4096;
 constexpr int kSharedCols = 16;           // columns of the 16x16x32 MFMA tile
-constexpr int kSharedWaves = 2048;        // shared-kernel wavefronts, all resident at D = 128
+constexpr int kSharedWaves = 2048;        // shared-kernel wavefronts at most; behind the split
+                                          // work's, with which they share the CUs
 
 struct SharedPlan {
     int32_t* nsub;      // [1] subgroups

@@ -403,8 +403,8 @@ __device__ __forceinline__ bf16x8 load_vt(const __bf16* lv, int h2, int n, int l
 }
 
 // Max growth (log2 units) tolerated before the accumulators are rescaled. Probabilities
-// stay <= 2^8 (pipelined kernel: below 2) and sums of them fit fp32 comfortably; acc and l always share one reference
-// max, so the final acc / l is exact whatever the reference.
+// stay <= 2^8 (pipelined kernel: below 2) and sums of them fit fp32 comfortably; acc and l
+// always share one reference max, so the final acc / l is exact whatever the reference.
 constexpr float kRescaleSlack = 8.0f;
 // Pipelined kernel: how far above a row's max the reference is set, so that probabilities
 // start at or below 2^-6 and the row may grow by 7 before one reaches 2.
@@ -748,15 +748,14 @@ __global__ __launch_bounds__(kThreads) void prefill_tile_kernel(
 // K and V tiles sit in rings of three in LDS, so one barrier per tile suffices and the first
 // operands of a tile's step are read before its barrier.
 //
-// What bounds it: the matrix pipe is busy 62 % of the cycles when half the CUs run (clock
-// 2.4 GHz), and the chip is power-limited (2.0-2.1 GHz) when all do. Left out one at a time in
-// copies of the kernel (1 x (12,345 cached + 1,024 new), 32q/8kv, 294 us then): LDS operand
-// reads -18 us, direct loads -20, barrier -13, row sums -14, exps -25; all but the MFMAs and
-// exps -58. Against the loop before (QK and PV in separate phases, row sums by
-// v_dot2_f32_bf16, row max in front of every exp, order left to the scheduler): that case
-// 312 -> 277 us (0.69 -> 0.78 PFLOP/s on 128 of 256 CUs), 8 x (8,192 + 1,024) 16q/8kv 548 ->
-// 518 us (1.07 -> 1.13), 8 x (512 + 1,536) 144.5 -> 141 us, head dim 64 8 x (4,096 + 1,024)
-// 350 -> 335 us, fp8 8 x (2,048 + 1,024) 195 -> 189 us.
+// What bounds it: the matrix pipe, at the clock that the chip's power limit leaves. Over a whole
+// launch it is busy 59 % of the cycles for 1 x (12,345 cached + 1,024 new) 32q/8kv (at 1.85 GHz)
+// and 46 % for 8 x (512 + 1,536) 16q/8kv (1.98 GHz; fewer key tiles a workgroup, so more of it is
+// prologue, masked tiles and tail); no LDS bank conflicts. Against the loop before (QK and PV in
+// separate phases, row sums by v_dot2_f32_bf16, row max in front of every exp, order left to the
+// scheduler), us a call with whole tiles: 1 x (12,345 + 1,024) 314 -> 276, 8 x (8,192 + 1,024)
+// 16q/8kv 561 -> 531 (1.04 -> 1.10 PFLOP/s), 8 x (512 + 1,536) 153 -> 146, head dim 64 32q/8kv
+// 8 x (4,096 + 1,024) 375 -> 346, fp8 16q/8kv 8 x (2,048 + 1,024) 209 -> 195.
 // ---------------------------------------------------------------------------
 __host__ __device__ constexpr bool pipe_head_dim(int d) { return d == 64 || d == 128; }
 
@@ -1738,6 +1737,8 @@ bool prefill_fp8_supported(int head_dim, int max_blocks_per_req) {
     return pipe_head_dim(head_dim) && max_blocks_per_req <= kMaxTableLds;
 }
 
+// Also for batches too large to split: a workspace sized for the largest call serves the smaller
+// ones, which do.
 size_t prefill_split_bytes(int head_dim, int max_blocks_per_req, int block_size) {
     const int D = decode_mfma_dim(head_dim);
     if (!pipe_head_dim(D) ||

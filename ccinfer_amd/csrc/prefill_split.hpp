@@ -10,24 +10,28 @@
 // under kSplitMinTiles. Each piece is a workgroup of its own that leaves unnormalised fp32 rows
 // and (m, l) pairs for the merge.
 //
-// A key tile takes ~1.8 us at head dim 128 (half that at 64), while a split costs the merge
-// (4-8 us) and a prologue per piece: tiles are split where that saves at least kSplitGain of
-// them. Whole -> split, us a call: 1 x (12,345 cached + 1,024 new) 32q/8kv 314 -> 208, 2 x (20,000
-// + 16) 451 -> 58, 1 x (2,000 + 512) 16q/8kv 72 -> 39, 1 x 2,048 16q/8kv 58 -> 40.5, 1 x (900 + 200)
-// 38 -> 22, 1 x (3,000 + 100) 32q/8kv head dim 64 62 -> 30. With 176-280 workgroups (2 x (1,000 cached + 700 new), 1 x 1,536 and 1 x 2,048 at 32q/8kv)
-// pieces of unequal rounds and the merge lost 6-8 us, hence the half; at savings of 8-12 key
-// tiles the two sides are even. An estimate of each of 16 piece lengths from a histogram of the
-// pieces, on the device, found little better lengths and took 5 us itself.
+// A key tile takes ~1.3 us at head dim 128 (half that at 64), while a split costs the merge
+// (4-10 us) and a prologue per piece: tiles are split where that saves at least kSplitGain of
+// them. Whole -> split, us a call replayed from a graph: 1 x (12,345 cached + 1,024 new) 32q/8kv
+// 276 -> 213, 2 x (20,000 + 16) 32q/8kv 396 -> 63, 1 x (2,000 + 512) 16q/8kv 68 -> 41, 1 x 2,048
+// 16q/8kv 56 -> 44, 1 x (900 + 200) 32q/8kv 36 -> 26, head dim 64 1 x (3,000 + 100) 32q/8kv
+// 56 -> 31, fp8 1 x (8,000 + 1,024) 32q/8kv 249 -> 164. With 176-280 workgroups (2 x (1,000 + 700),
+// 1 x 1,536 and 1 x 2,048 at 32q/8kv) pieces of unequal rounds and the merge lost 6-8 us, hence
+// the half; at savings of 8-12 key tiles the two sides are even. An estimate of each of 16 piece
+// lengths from a histogram of the pieces, on the device, found little better lengths and took
+// 5 us itself.
 //
 // The host knows the widths of the table rows, not the lengths, so it can only tell that a launch
 // may split (SplitRule); most such launches of short prompts over wide tables do not. The lengths
 // are read where they are used: every wavefront of a tile workgroup and of the merge derives the
 // plan from query_start_loc and context_lens, one request a lane, and no list is kept. At up to
-// 2,048 positions such a launch needs no planner, which pays for the merge: 1 x 200 new tokens on
-// a table of 128 blocks 17.4 us without splits, 15.3 now (20.6 with pieces listed by the planner).
-// Wider tables need it for the decode items, whose merge then takes the tiles' along: 1 x 200 on
-// 2,048 blocks 20.6 without splits, 22.0 now (23.3 with a list and a merge launch of its own); 1.1
-// of the 1.4 are the tile kernel's, not the split's. An in-launch merge by the last piece would
+// 2,048 positions such a launch needs no planner, which pays for the merge: 16q/8kv on a table of
+// 128 blocks, without splits -> now, 1 x 200 new tokens 18.1 -> 15.0 us, 8 x 200 19.8 -> 16.5.
+// Wider tables need it for the decode items, whose merge then takes the tiles' along: on 2,048
+// blocks 1 x 200 21.3 -> 22.0, 8 x 200 22.9 -> 24.6, 4 x 200 with four single-token requests
+// 27.5 -> 28.9 (the merge now comes after the tiles, with a wavefront per possible row). A word of
+// the planner that spares both the plan where nothing splits took 0.3-0.9 us off these and cost
+// every other prompt 0.2-0.4 (the tile kernel's start). An in-launch merge by the last piece would
 // need agent-scope fences, which write back and invalidate the L2.
 #pragma once
 
@@ -161,8 +165,9 @@ __device__ __forceinline__ bool split_piece(const SplitRule& a, const SplitPlan&
     const int len = __builtin_amdgcn_readfirstlane(cost / c);
     const int more = cost - len * c;
     const int kt0 = k * len + min(k, more);
-    *out = TilePiece{b, __builtin_amdgcn_readlane(s.qb, b), rows, prefix, t0, kt0, kt0 + len + (k < more ? 1 : 0),
-                     tile * s.per + k, c};
+    const int kt1 = kt0 + len + (k < more ? 1 : 0);
+    const int qb = __builtin_amdgcn_readlane(s.qb, b);
+    *out = TilePiece{b, qb, rows, prefix, t0, kt0, kt1, tile * s.per + k, c};
     return true;
 }
 
@@ -188,8 +193,9 @@ inline int tile_merge_wgs(const TileMerge& t, int D) {
 // wavefront of the tile kernel, 32-dim block n): it reads the partials in the tile kernel's own
 // lane layout, so every load is a whole kilobyte, and stores the rows as that kernel's epilogue
 // does. Wavefronts of tiles that are whole, or not there, leave at once. Bound by the latency of
-// its loads: with the pieces of a batch loaded together, 2 x (20,000 + 16) 64.5 -> 58 us a call
-// against a loop left to the scheduler (8 pieces at a time: 58; 1 x 2,048, two pieces, 40.5 -> 42).
+// its loads: with the pieces of a batch loaded together, 2 x (20,000 + 16) takes 10 % less a call
+// than with a loop left to the scheduler (8 pieces at a time: the same; 1 x 2,048, whose tiles have
+// two pieces, then 4 % more).
 template <int D, bool kPad>
 __device__ __forceinline__ void merge_tile_pieces(const TileMerge& t, int wi) {
     constexpr int kPipeWaves = PipeShape<D>::kWaves;

@@ -234,9 +234,10 @@ int ccinfer_decode_attention_fp8(const void* q, const void* k_cache, const void*
 /* Workspace bytes ccinfer_prefill_attention (and the fp8 / overlap variants) needs for this
  * batch shape; 0 for invalid shapes. As for decode, it includes two copies of
  * the q rows used only by a call with a 2-byte-aligned q or output. It also includes the
- * memory (17-34 MB at head dims up to 128, table rows past ~1,100 positions) in which a batch that fills at most half the GPU
- * keeps the partial rows of its query tiles, whose key ranges it splits over more workgroups;
- * a call given a workspace that much smaller is accepted and runs its tiles whole. */
+ * memory in which a batch that fills at most half the GPU keeps the partial rows of its query
+ * tiles, whose key ranges it splits over more workgroups (head dims up to 64: 17 MB where a table
+ * row holds more than 1,984 positions; up to 128: 34 MB, more than 1,088); a call given a
+ * workspace that much smaller is accepted and runs its tiles whole. */
 size_t ccinfer_prefill_workspace_size(int batch_size, int total_query_tokens,
                                       int max_blocks_per_req, int num_q_heads,
                                       int num_kv_heads, int head_dim, int cache_block_size);
